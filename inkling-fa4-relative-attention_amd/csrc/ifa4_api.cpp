@@ -172,6 +172,10 @@ ifa4::PrefillParams make_prefill_params(const ifa4_args* a) {
   p.scale_log2 = a->softmax_scale * kLog2eHost;
   p.chunk_tiles = 0;
   p.n_chunks = 1;
+  // lengths a sixteenth below the longest on average: the ragged workgroup order
+  // (8 x 3990..4090 tokens, 1% below, run 2% slower in it)
+  p.ragged = 16 * a->total_q < (int64_t)15 * a->batch * a->max_seqlen_q ||
+             16 * a->total_k < (int64_t)15 * a->batch * a->max_seqlen_k;
   return p;
 }
 
