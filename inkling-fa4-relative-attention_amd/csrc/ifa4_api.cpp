@@ -179,6 +179,15 @@ ifa4::PrefillParams make_prefill_params(const ifa4_args* a) {
   return p;
 }
 
+ifa4::PrefillSplit prefill_split(const ifa4_args* a) {
+  return ifa4::prefill_split_for(a->batch, a->n_heads, a->max_seqlen_q, a->max_seqlen_k,
+                                 a->causal != 0, a->window_left,
+                                 (a->flags & IFA4_FLAG_BOTTOM_RIGHT) != 0,
+                                 (a->flags & IFA4_FLAG_NO_PRUNE) != 0, ifa4::prefill_block_q(),
+                                 ifa4::prefill_block_k(),
+                                 (a->flags & IFA4_FLAG_SPLIT_KV_2) ? 2 : 0);
+}
+
 // Split-KV plan of a prefill call and the workspace it needs: partial O
 // [n_chunks][n_heads][total_q][head_dim] fp32, then their LSEs, 256-byte aligned.
 struct PrefillWorkspace {
@@ -188,14 +197,7 @@ struct PrefillWorkspace {
 };
 PrefillWorkspace prefill_workspace(const ifa4_args* a) {
   PrefillWorkspace w;
-  const bool bottom_right = (a->flags & IFA4_FLAG_BOTTOM_RIGHT) != 0;
-  // bottom-right masks see the last max_seqlen_q keys' positions: estimate with
-  // the full key range visible (causal off), which only shifts the heuristic
-  w.split = ifa4::prefill_split_for(a->batch, a->n_heads, a->max_seqlen_q, a->max_seqlen_k,
-                                    a->causal != 0 && !bottom_right,
-                                    bottom_right ? -1 : a->window_left, ifa4::prefill_block_q(),
-                                    ifa4::prefill_block_k(),
-                                    (a->flags & IFA4_FLAG_SPLIT_KV_2) ? 2 : 0);
+  w.split = prefill_split(a);
   const int64_t rows = (int64_t)w.split.n_chunks * a->n_heads * a->total_q;
   w.o_bytes = (rows * a->head_dim * 4 + 255) / 256 * 256;
   w.lse_bytes = (rows * 4 + 255) / 256 * 256;
@@ -380,11 +382,7 @@ int32_t ifa4_prefill_tile(const ifa4_args* args, ifa4_tile* tile) {
       tile->waves = e.waves;
       tile->stages = e.stages;
       // split KV (ifa4_prefill_fwd_ws): keys per chunk, 0 when the call does not split
-      const ifa4::PrefillSplit sp = ifa4::prefill_split_for(
-          args->batch, args->n_heads, args->max_seqlen_q, args->max_seqlen_k,
-          args->causal != 0 && (args->flags & IFA4_FLAG_BOTTOM_RIGHT) == 0,
-          (args->flags & IFA4_FLAG_BOTTOM_RIGHT) ? -1 : args->window_left, e.block_q, e.block_k,
-          (args->flags & IFA4_FLAG_SPLIT_KV_2) ? 2 : 0);
+      const ifa4::PrefillSplit sp = prefill_split(args);
       tile->kv_chunk = sp.chunk_tiles * e.block_k;
       return IFA4_OK;
     }
