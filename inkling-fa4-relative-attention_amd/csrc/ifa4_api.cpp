@@ -132,6 +132,16 @@ int32_t check_paged(const ifa4_args* a, const ifa4_paged_kv* kv, int kv_esize = 
   return IFA4_OK;
 }
 
+// Query tiles of block_q rows, `pack` query heads of a kv head side by side.
+void set_tiles(ifa4::PrefillParams& p, const ifa4_args* a, int block_q, int pack) {
+  p.pack = pack;
+  p.q_step = block_q / pack;
+  p.pack_magic = (65536 + pack - 1) / pack;
+  p.tile_heads = a->n_heads / pack;
+  p.tile_group = a->n_heads / a->kv_heads / pack;
+  p.n_qtiles = (int)(((int64_t)a->max_seqlen_q + p.q_step - 1) / p.q_step);
+}
+
 ifa4::PrefillParams make_prefill_params(const ifa4_args* a) {
   ifa4::PrefillParams p{};
   p.q = a->q;
@@ -167,11 +177,12 @@ ifa4::PrefillParams make_prefill_params(const ifa4_args* a) {
   p.bottom_right = (a->flags & IFA4_FLAG_BOTTOM_RIGHT) ? 1 : 0;
   p.no_prune = (a->flags & IFA4_FLAG_NO_PRUNE) ? 1 : 0;
   p.rel_dtype = a->rel_dtype;
-  const int bq = ifa4::prefill_block_q();
-  p.n_qtiles = (a->max_seqlen_q + bq - 1) / bq;
   p.scale_log2 = a->softmax_scale * kLog2eHost;
   p.chunk_tiles = 0;
   p.n_chunks = 1;
+  p.seen_chunks = 1;
+  p.max_q = a->max_seqlen_q;
+  set_tiles(p, a, ifa4::prefill_block_q(), 1);
   // lengths a sixteenth below the longest on average: the ragged workgroup order
   // (8 x 3990..4090 tokens, 1% below, run 2% slower in it)
   p.ragged = 16 * a->total_q < (int64_t)15 * a->batch * a->max_seqlen_q ||
@@ -179,25 +190,49 @@ ifa4::PrefillParams make_prefill_params(const ifa4_args* a) {
   return p;
 }
 
-ifa4::PrefillSplit prefill_split(const ifa4_args* a) {
-  return ifa4::prefill_split_for(a->batch, a->n_heads, a->max_seqlen_q, a->max_seqlen_k,
+// Query heads of a kv head whose rows share the query tiles: the whole group
+// when that takes fewer tiles (prefill_packs), and its q rows and bias rows stay
+// below the 2 GiB of a buffer resource (a shared bias table: its copies below
+// the LDS they get); else one.
+int prefill_pack(const ifa4_args* a) {
+  const int64_t kLimit = int64_t(1) << 31;
+  const int64_t group = a->n_heads / a->kv_heads;
+  const int bq = ifa4::prefill_block_q();
+  if (!ifa4::prefill_packs(group, a->max_seqlen_q, bq)) return 1;
+  const int64_t rows = (int64_t)a->max_seqlen_q + bq;
+  const int64_t esize = a->rel_dtype == IFA4_FP32 ? 4 : 2;
+  if ((rows * a->q_stride_t + (group - 1) * a->q_stride_h + a->head_dim) * 2 >= kLimit) return 1;
+  if (a->rel_extent > 0 &&
+      (rows * a->rel_stride_t + (group - 1) * a->rel_stride_h + a->rel_width) * esize >= kLimit)
+    return 1;
+  ifa4::PrefillParams p{};
+  p.rel_st = a->rel_stride_t;
+  p.rel_extent = a->rel_extent;
+  if (ifa4::prefill_tab(p) && !ifa4::prefill_tab_packs(a->rel_extent, (int)group)) return 1;
+  return (int)group;
+}
+
+ifa4::PrefillSplit prefill_split(const ifa4_args* a, int pack) {
+  return ifa4::prefill_split_for(a->batch, a->n_heads / pack, a->max_seqlen_q, a->max_seqlen_k,
                                  a->causal != 0, a->window_left,
                                  (a->flags & IFA4_FLAG_BOTTOM_RIGHT) != 0,
-                                 (a->flags & IFA4_FLAG_NO_PRUNE) != 0, ifa4::prefill_block_q(),
-                                 ifa4::prefill_block_k(),
+                                 (a->flags & IFA4_FLAG_NO_PRUNE) != 0,
+                                 ifa4::prefill_block_q() / pack, ifa4::prefill_block_k(),
                                  (a->flags & IFA4_FLAG_SPLIT_KV_2) ? 2 : 0);
 }
 
 // Split-KV plan of a prefill call and the workspace it needs: partial O
 // [n_chunks][n_heads][total_q][head_dim] fp32, then their LSEs, 256-byte aligned.
 struct PrefillWorkspace {
+  int pack;
   ifa4::PrefillSplit split;
   int64_t o_bytes, lse_bytes;
   int64_t total() const { return split.chunk_tiles > 0 ? o_bytes + lse_bytes : 0; }
 };
 PrefillWorkspace prefill_workspace(const ifa4_args* a) {
   PrefillWorkspace w;
-  w.split = prefill_split(a);
+  w.pack = prefill_pack(a);
+  w.split = prefill_split(a, w.pack);
   const int64_t rows = (int64_t)w.split.n_chunks * a->n_heads * a->total_q;
   w.o_bytes = (rows * a->head_dim * 4 + 255) / 256 * 256;
   w.lse_bytes = (rows * 4 + 255) / 256 * 256;
@@ -382,7 +417,7 @@ int32_t ifa4_prefill_tile(const ifa4_args* args, ifa4_tile* tile) {
       tile->waves = e.waves;
       tile->stages = e.stages;
       // split KV (ifa4_prefill_fwd_ws): keys per chunk, 0 when the call does not split
-      const ifa4::PrefillSplit sp = prefill_split(args);
+      const ifa4::PrefillSplit sp = prefill_split(args, 1);
       tile->kv_chunk = sp.chunk_tiles * e.block_k;
       return IFA4_OK;
     }
@@ -412,11 +447,13 @@ int32_t ifa4_prefill_fwd_ws(const ifa4_args* args, void* workspace, size_t works
   if (args->batch == 0 || args->max_seqlen_q == 0) return IFA4_OK;
   ifa4::PrefillParams p = make_prefill_params(args);
   const PrefillWorkspace w = prefill_workspace(args);
+  set_tiles(p, args, ifa4::prefill_block_q(), w.pack);
   if (w.total() > 0) {
     if (workspace == nullptr || workspace_bytes < (size_t)w.total() || !aligned(workspace, 256))
       return IFA4_EWORKSPACE;
     p.chunk_tiles = w.split.chunk_tiles;
     p.n_chunks = w.split.n_chunks;
+    p.seen_chunks = w.split.seen_chunks;
     p.part_o = static_cast<float*>(workspace);
     p.part_lse = reinterpret_cast<float*>(static_cast<char*>(workspace) + w.o_bytes);
   }
@@ -455,8 +492,7 @@ int32_t ifa4_prefill_rproj_fwd(const ifa4_args* args, const ifa4_rel_proj* pr, v
   p.rel_sh = pr->r_stride_h;
   p.wt = args->rel_extent > 0 ? pr->wt : nullptr;  // no bias at all: the plain kernel
   if (p.wt != nullptr) {
-    const int bq = ifa4::prefill_proj_block_q();
-    p.n_qtiles = (args->max_seqlen_q + bq - 1) / bq;
+    set_tiles(p, args, ifa4::prefill_proj_block_q(), 1);
   }
   const hipError_t e = ifa4::launch_prefill(p, args->head_dim, args->qkv_dtype,
                                             static_cast<hipStream_t>(stream));

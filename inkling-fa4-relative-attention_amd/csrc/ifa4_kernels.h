@@ -47,6 +47,12 @@ struct PrefillParams {
   // units) part_lse [n_chunks][n_heads][total_q], merged by a second pass.
   int32_t chunk_tiles;
   int32_t n_chunks;
+  int32_t seen_chunks;  // slots that pruned query tiles can use (the merge's form)
+  // A query tile is q_step queries x `pack` query heads of one kv head (packed
+  // rows, pack > 1: row r of the tile is query (r * pack_magic) >> 16); tile_heads
+  // = n_heads / pack tiles side by side, tile_group of them per kv head.
+  int32_t pack, q_step, pack_magic, tile_heads, tile_group;
+  int32_t max_q;        // max_seqlen_q
   float* part_o;
   float* part_lse;
   // Fused relative-logit projection (wt != nullptr): rel / rel_st / rel_sh /
@@ -100,6 +106,8 @@ struct DecodeParams {
 int prefill_block_q();
 int prefill_proj_block_q();  // query rows per workgroup of the fused-projection kernel
 int prefill_block_k();
+bool prefill_tab(const PrefillParams& p);  // the shared bias table is staged in LDS
+bool prefill_tab_packs(int rel_extent, int pack);  // ... and holds the tables of `pack` heads
 int prefill_waves();
 hipError_t launch_prefill(const PrefillParams& p, int head_dim, int qkv_dtype, hipStream_t stream);
 

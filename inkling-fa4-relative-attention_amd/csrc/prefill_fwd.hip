@@ -95,12 +95,6 @@
 #ifndef IFA4_MERGE_BATCH
 #define IFA4_MERGE_BATCH 4
 #endif
-#ifndef IFA4_MERGE_PARTS
-#define IFA4_MERGE_PARTS 8
-#endif
-#ifndef IFA4_MERGE_THREADS
-#define IFA4_MERGE_THREADS 256
-#endif
 
 namespace ifa4 {
 namespace {
@@ -188,6 +182,12 @@ constexpr int vmcnt_imm(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >>
 constexpr int kLgkm0 = 15 | (7 << 4) | (0 << 8) | (3 << 14);
 
 constexpr int kBiasLdsMax = 1024;  // longest shared bias table staged in LDS
+// Packed rows: LDS for the tables of all packed heads (16 KiB beside the two 32
+// KiB stages at d 128, so that two workgroups still share a CU).
+constexpr int kBiasPackFloats = 4096;
+__host__ __device__ constexpr int bias_pack_pitch(int rel_extent, int pack, int pad) {
+  return (rel_extent + 2 * pad + 31) / 32 * 32 + (pack > 1 ? (pack < 32 ? 32 / pack : 1) : 0);
+}
 
 // Fused relative-logit projection (kProj): bias(i, dist) = sum_c r[i, c] *
 // W[c, dist] with r [Tq, Hq, kProjDim] and W^T [R', kProjDim] fp32, any
@@ -227,7 +227,7 @@ __device__ __forceinline__ uint32_t span_bytes(int rows, int64_t stride, int d, 
   return rows > 0 ? (uint32_t)(((int64_t)(rows - 1) * stride + d) * esize) : 0u;
 }
 
-// KV tiles [kt_beg, kt_end) a query tile visits (tile pruning): causal keeps
+// KV tiles [kt_beg, kt_end) the query tile [q0, q_hi) visits (tile pruning): causal keeps
 // keys below the tile's last row (+ qpos), the window keys from its first row
 // (+ qpos) minus window_left; the prefill kernel and the merge of split-KV
 // partials both derive a tile's range (and so its chunk count) from this.
@@ -235,9 +235,8 @@ struct TileRange {
   int beg, end;
 };
 template <typename Sh>
-__device__ __forceinline__ TileRange tile_range(const PrefillParams& p, int q0, int lq, int lk,
+__device__ __forceinline__ TileRange tile_range(const PrefillParams& p, int q0, int q_hi, int lk,
                                                 int qpos) {
-  const int q_hi = min(q0 + Sh::kBlockQ, lq);  // exclusive
   int kend = lk, kbeg = 0;
   if (!p.no_prune) {
     if (p.causal) kend = min(kend, q_hi + qpos);
@@ -260,17 +259,49 @@ __device__ __forceinline__ int tile_chunks(const PrefillParams& p, const TileRan
   return min(max(n, 1), p.n_chunks);
 }
 
-template <typename Sh, int D, typename Tag, typename Rel, bool kProj, bool kTab>
-__global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
-    Sh::kWavesPerSimd, Sh::kWavesPerSimd))) void prefill_fwd_kernel(PrefillParams p) {
+// Query of row r of a packed item, from the item's first (r < 256).
+__device__ __forceinline__ int packed_query(const PrefillParams& p, int r) {
+  return (int)(((uint32_t)r * (uint32_t)p.pack_magic) >> 16);
+}
+
+// One piece of work of a workgroup: a block of query rows and a range of KV tiles.
+struct WorkItem {
+  int qs, lq, ks, lk;  // the sequence's first row and length in q / out and in k / v
+  int qpos, delta;     // query i sits at key position i + qpos; dist = i + delta - j
+  int kvh, head0;      // kv head, first query head
+  int q0, q_end;       // queries [q0, q_end) of the sequence
+  int kt_beg, kt_end;  // KV tiles
+  int part;            // KV chunk of a split query block, or -1
+};
+
+// Query i sits at key position i + qpos for the causal and window masks;
+// the bias distance is dist = i + delta - j.  Top-left (the reference
+// oracle, src/inkling_fa4/reference.py:28-37): qpos = 0, delta = lq - lk.
+// Bottom-right (upstream flash-attn): qpos = delta = lk - lq.
+__device__ __forceinline__ void set_sequence(const PrefillParams& p, WorkItem& it, int seq) {
+  const SeqBounds bq = seq_bounds(p.cu_q, seq, p.total_q);
+  const SeqBounds bk = seq_bounds(p.cu_k, seq, p.total_k);
+  it.qs = bq.start;
+  it.lq = bq.len;
+  it.ks = bk.start;
+  it.lk = bk.len;
+  it.qpos = p.bottom_right ? bk.len - bq.len : 0;
+  it.delta = p.bottom_right ? bk.len - bq.len : bq.len - bk.len;
+}
+
+// Attention of one work item.  kPack: the rows are packed, row r of the item is
+// query q0 + r / pack, query head head0 + r % pack (p.pack query heads of one kv
+// head side by side); otherwise the rows are queries of head0.
+template <typename Sh, int D, typename Tag, typename Rel, bool kProj, bool kTab, bool kPack>
+__device__ __forceinline__ void prefill_work(const PrefillParams& p, const WorkItem& it) {
   using E = Elem<Tag>;
   using St = PrefillStage<Sh, D>;
-  constexpr int kNqb = Sh::kNqb, kBlockQ = Sh::kBlockQ;
+  constexpr int kNqb = Sh::kNqb;
   constexpr int kBlockK = Sh::kBlockK, kThreads = Sh::kThreads, kBiasPad = Sh::kBiasPad;
-  constexpr int kBiasLdsFloats = 2 * kBiasPad + kBiasLdsMax;
-  constexpr int kBiasTop = kBiasLdsMax + kBiasPad - 1;  // table index of dist 0
+  constexpr int kBiasLdsFloats = kPack ? kBiasPackFloats : 2 * kBiasPad + kBiasLdsMax;
   constexpr int kDBlocks = D / 32;
   constexpr int kKSteps = D / 16;
+  static_assert(!kPack || kNqb == 1, "packed rows: one row block per wave");
 
   // Both stages in one array: a read of stage 1 is the stage-0 address plus a
   // constant, which folds into the instruction's offset (one address register
@@ -284,65 +315,13 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
   uint16_t* const stage0 = stages;
   uint16_t* const stage1 = stages + St::kElems;
 
-  // ---- which (q tile, KV chunk, head, sequence): heaviest (last) q tiles first --
-  // A q tile's chunks (split KV; one when not splitting) are consecutive, so
-  // a chunk that ends early is followed by the next q tile's work.
-  int qtile, chunk, head, seq;
-  if (p.xcd_spread) {  // ragged (prefill_order)
-    const int x = blockIdx.x & 7;
-    int slot = blockIdx.x >> 3;
-    const int m = slot % p.xcd_unit;
-    slot /= p.xcd_unit;
-    const int k = slot % p.xcd_heads;
-    slot /= p.xcd_heads;
-    const int rounds = (p.batch + p.xcd_spread - 1) / p.xcd_spread;
-    const int qc = slot / rounds;
-    seq = (slot + qc) % rounds * p.xcd_spread + ((x + 7 * qc) & (p.xcd_spread - 1));
-    if (seq >= p.batch) return;
-    head = (p.xcd_spread > 1 ? x / p.xcd_spread : x * p.xcd_heads + k) * p.xcd_unit + m;
-    qtile = p.n_qtiles - 1 - qc / p.n_chunks;
-    chunk = qc % p.n_chunks;
-  } else if (p.xcd_pairs) {
-    // Workgroup i runs on XCD i % 8.  Give XCD x the (sequence, kv head) pairs
-    // x, x+8, ... so their K/V stay in that XCD's L2; heaviest q tiles first.
-    const int x = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    const int per_xcd = p.xcd_pairs;  // pairs per XCD
-    const int per_tile = per_xcd * p.group;
-    const int qc = slot / per_tile;
-    qtile = p.n_qtiles - 1 - qc / p.n_chunks;
-    chunk = qc % p.n_chunks;
-    const int rem = slot % per_tile;
-    const int pair = x + 8 * (rem / p.group);
-    const int kv_heads = p.n_heads / p.group;
-    seq = pair / kv_heads;
-    head = (pair % kv_heads) * p.group + rem % p.group;
-  } else {
-    const int per_tile = p.n_heads * p.batch;
-    const int lin = blockIdx.x;
-    const int qc = lin / per_tile;
-    qtile = p.n_qtiles - 1 - qc / p.n_chunks;
-    chunk = qc % p.n_chunks;
-    const int rem = lin % per_tile;
-    head = rem % p.n_heads;
-    seq = rem / p.n_heads;
-    if (p.ragged) seq = (seq + qc) % p.batch;
-  }
-
-  const SeqBounds bq = seq_bounds(p.cu_q, seq, p.total_q);
-  const SeqBounds bk = seq_bounds(p.cu_k, seq, p.total_k);
-  const int qs = bq.start, lq = bq.len;
-  const int ks = bk.start, lk = bk.len;
-  const int q0 = qtile * kBlockQ;
-  if (q0 >= lq) return;
-  const int kvh = head / p.group;
-  // Query i sits at key position i + qpos for the causal and window masks;
-  // the bias distance is dist = i + delta - j.  Top-left (the reference
-  // oracle, src/inkling_fa4/reference.py:28-37): qpos = 0, delta = lq - lk.
-  // Bottom-right (upstream flash-attn): qpos = delta = lk - lq.
-  const int qpos = p.bottom_right ? lk - lq : 0;
-  const int delta = p.bottom_right ? lk - lq : lq - lk;
+  const int qs = it.qs, lq = it.lq, ks = it.ks, lk = it.lk;
+  const int q0 = it.q0, kvh = it.kvh, head = it.head0;
+  const int qpos = it.qpos, delta = it.delta;
+  const int kt_beg = it.kt_beg, kt_end = it.kt_end;
   const int wl = p.window_left;
   const int rext = p.rel_extent;
+  const int pack = kPack ? p.pack : 1;
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
@@ -357,36 +336,34 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
                            (int64_t)kvh * p.k_sh;
   const uint16_t* v_base = static_cast<const uint16_t*>(p.v) + (int64_t)ks * p.v_st +
                            (int64_t)kvh * p.v_sh;
-  const rsrc_t rq = make_rsrc(q_base, span_bytes(lq, p.q_st, D, 2));
+  const rsrc_t rq =
+      make_rsrc(q_base, span_bytes(lq, p.q_st, D + (pack - 1) * (int)p.q_sh, 2));
   [[maybe_unused]] const rsrc_t rk = make_rsrc(k_base, span_bytes(lk, p.k_st, D, 2));
   [[maybe_unused]] const rsrc_t rv = make_rsrc(v_base, span_bytes(lk, p.v_st, D, 2));
   const uint32_t k_row = (uint32_t)p.k_st * 2, v_row = (uint32_t)p.v_st * 2;
 
-  // ---- key range of the workgroup (tile pruning, then this KV chunk) ---------
-  const TileRange tr = tile_range<Sh>(p, q0, lq, lk, qpos);
-  const int nch = tile_chunks(p, tr);
-  if (chunk >= nch) return;
-  int kt_beg = tr.beg, kt_end = tr.end;
-  if (nch > 1) {
-    const int c0 = (tr.beg / p.chunk_tiles + chunk) * p.chunk_tiles;
-    kt_beg = max(tr.beg, c0);
-    kt_end = min(tr.end, c0 + p.chunk_tiles);
-  }
-
   // ---- per-wave rows ---------------------------------------------------------
-  const int qa = q0 + 32 * kNqb * wave;                  // first row of the wave (local)
-  const int wrows = max(0, min(32 * kNqb, lq - qa));     // valid rows of the wave
+  // queries [imin, imax] of this wave's rows (none: imin > imax)
+  const int row0 = 32 * kNqb * wave;
+  const int imin = q0 + (kPack ? packed_query(p, row0) : row0);
+  const int imax =
+      min(q0 + (kPack ? packed_query(p, row0 + 32 * kNqb - 1) : row0 + 32 * kNqb - 1), it.q_end - 1);
+  const bool live = imin <= imax;
   int wkend = lk, wkbeg = 0;
   if (!p.no_prune) {
-    if (p.causal) wkend = min(lk, qa + wrows + qpos);
-    if (wl >= 0) wkbeg = max(0, qa + qpos - wl);
+    if (p.causal) wkend = min(lk, imax + 1 + qpos);
+    if (wl >= 0) wkbeg = max(0, imin + qpos - wl);
   }
   int qi[kNqb];        // this lane's query (local) in each row block
+  int hq[kNqb];        // and its query head, from head0
   bool row_ok[kNqb];
 #pragma unroll
   for (int qb = 0; qb < kNqb; ++qb) {
-    qi[qb] = qa + 32 * qb + col;
-    row_ok[qb] = qi[qb] < lq;
+    const int r = row0 + 32 * qb + col;
+    const int ql = kPack ? packed_query(p, r) : r;
+    qi[qb] = q0 + ql;
+    hq[qb] = kPack ? r - ql * pack : 0;
+    row_ok[qb] = qi[qb] < it.q_end;
   }
 
   // ---- Q fragments (B operand), kept for the whole loop ----------------------
@@ -394,8 +371,11 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
   for (int qb = 0; qb < kNqb; ++qb)
 #pragma unroll
-    for (int kk = 0; kk < kKSteps; ++kk)
-      qf[qb][kk] = buf_load_16(rq, (uint32_t)(qi[qb] * p.q_st + 16 * kk + 8 * half) * 2);
+    for (int kk = 0; kk < kKSteps; ++kk) {
+      const uint32_t off =
+          (uint32_t)(qi[qb] * (int)p.q_st + hq[qb] * (int)p.q_sh + 16 * kk + 8 * half) * 2;
+      qf[qb][kk] = buf_load_16(rq, !kPack || row_ok[qb] ? off : kOutOfRange);
+    }
 
   const float c2 = p.scale_log2;  // softmax_scale * log2(e)
   const float inv_scale = kLog2e / c2;  // bias -> score units (1 / softmax_scale)
@@ -473,11 +453,18 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
   const rsrc_t rrel = make_rsrc(
       static_cast<const char*>(p.rel) + ((int64_t)qs * p.rel_st + (int64_t)head * p.rel_sh) *
                                             Rel::kBytes,
-      span_bytes(lq, p.rel_st, kProj ? kProjDim : p.rel_width, Rel::kBytes));
+      span_bytes(lq, p.rel_st,
+                 (kProj ? kProjDim : p.rel_width) + (pack - 1) * (int)p.rel_sh, Rel::kBytes));
   // Shared-table layout with a table short enough to stage in LDS (the host
   // launches the kTab instantiation for it: token stride 0, rel_extent <=
   // kBiasLdsMax); the other instantiation reads per-token rows.
   const bool bias_in_lds = kTable && rext > 0;
+  // Table index of dist 0, entries and pitch of one head's table.  Packed rows
+  // hold pack tables; the pitch puts the heads of one query 32 / pack banks
+  // apart, so a wave's rows (32 / pack queries x pack heads) read distinct banks.
+  const int tab_top = kPack ? rext + kBiasPad - 1 : kBiasLdsMax + kBiasPad - 1;
+  const int tab_len = kPack ? rext + 2 * kBiasPad : kBiasLdsFloats;
+  [[maybe_unused]] const int tab_pitch = kPack ? bias_pack_pitch(rext, pack, kBiasPad) : 0;
   // Fused projection.  W^T [rel_width, 16] fp32 (64-byte rows) stays in L2;
   // rows outside [0, rel_extent) read as zero, so the projected bias is zero
   // there with no further test.  The B operand (this lane's row of r, channels
@@ -489,18 +476,18 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
   u32x4_t w_raw[3][2];
   // wave-uniform: the tile at kb is visited by this wave and meets the band
   auto proj_tile = [&](int kb) {
-    return rext > 0 && wrows > 0 && kb < wkend && kb + kBlockK > wkbeg &&
-           qa + wrows - 1 + delta - kb >= 0 && qa + delta - (kb + kBlockK - 1) <= rext - 1;
+    return rext > 0 && live && kb < wkend && kb + kBlockK > wkbeg &&
+           imax + delta - kb >= 0 && imin + delta - (kb + kBlockK - 1) <= rext - 1;
   };
   // distance block t of the tile at kb meets [0, rext) (wave-uniform); blocks
   // that do not are zero and skip their fetch and products
   auto proj_live = [&](int kb, int t) {
-    const int lo = qa + delta - kb - (kBlockK - 1) + 32 * t;
+    const int lo = imin + delta - kb - (kBlockK - 1) + 32 * t;
     return !IFA4_PROJ_SKIP || (lo + 31 >= 0 && lo < rext);
   };
   auto proj_fetch = [&](int kt) {
     if (!proj_tile(kt * kBlockK)) return;
-    const int d0 = qa + delta - kt * kBlockK - (kBlockK - 1) + col;  // block 0, row col
+    const int d0 = imin + delta - kt * kBlockK - (kBlockK - 1) + col;  // block 0, row col
 #pragma unroll
     for (int t = 0; t < 3; ++t) {
       if (!proj_live(kt * kBlockK, t)) continue;
@@ -549,7 +536,7 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
   constexpr bool kProjEarly = IFA4_PROJ_EARLY;
   auto proj_bias = [&](int kb, int blk, float* bias) {
     if (!(kProjEarly && blk == 0)) proj_fill(kb, blk);
-    const float* src = mp + col * (kProjPitch + 1) + 31 - 16 * half;
+    const float* src = mp + col * kProjPitch + (qi[0] - imin) + 31 - 16 * half;
 #pragma unroll
     for (int e = 0; e < 16; ++e) bias[e] = src[-e];
   };
@@ -567,7 +554,14 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
                                                 ((int64_t)qs * p.rel_st + (int64_t)head * p.rel_sh) *
                                                     Rel::kBytes) >> 1) & 1
                                        : 0;  // element parity of the resource base
-  const int rel_span = lq > 0 ? (lq - 1) * (int)p.rel_st + p.rel_width : 0;  // elements
+  const int rel_span =  // elements
+      lq > 0 ? (lq - 1) * (int)p.rel_st + (pack - 1) * (int)p.rel_sh + p.rel_width : 0;
+  // element offset of the lane's bias row in row block qb
+  int rel_row0[kNqb];
+#pragma unroll
+  for (int qb = 0; qb < kNqb; ++qb)
+    rel_row0[qb] = kPack ? qi[qb] * (int)p.rel_st + hq[qb] * (int)p.rel_sh : 0;
+  auto rel_row_of = [&](int qb) { return kPack ? rel_row0[qb] : qi[qb] * (int)p.rel_st; };
   auto token_bias = [&](int rel_row, int dtop, bool valid, float* bias) {
     constexpr int kSpan = Rel::kBytes == 2 ? 18 : 16;  // elements the vector loads cover
     const int lo = rel_row + dtop - 15;               // element of the lowest distance
@@ -717,7 +711,7 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
   auto compute = [&](int kt, const uint16_t* stage) {
     const int kb = kt * kBlockK;
     // Wave-uniform activity / class of this tile.
-    const bool active = wrows > 0 && kb < wkend && kb + kBlockK > wkbeg;
+    const bool active = live && kb < wkend && kb + kBlockK > wkbeg;
     // W^T rows of the next tile (fused projection): fetched once this tile's
     // are consumed, so that only one tile's operands are live at a time
     auto fetch_next = [&] {
@@ -728,7 +722,6 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
       fetch_next();
       return;
     }
-    const int imin = qa, imax = qa + wrows - 1;
     const int jmin = kb, jmax = kb + kBlockK - 1;
     const bool need_mask = jmax >= lk || (p.causal && jmax > imin + qpos) ||
                            (wl >= 0 && imax + qpos - jmin > wl);
@@ -749,7 +742,7 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
         for (int qb = 0; qb < kNqb; ++qb)
 #pragma unroll
           for (int blk = 0; blk < kBlockK / 32; ++blk)
-            tok_issue(qi[qb] * (int)p.rel_st, qi[qb] + delta - kb - 16 * half - 32 * blk,
+            tok_issue(rel_row_of(qb), qi[qb] + delta - kb - 16 * half - 32 * blk,
                       row_ok[qb], traw[qb][blk]);
         asm volatile("" ::: "memory");  // keep them ahead of the products
       }
@@ -828,15 +821,15 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
       const int dbase = qi[qb] + delta - kb - 16 * half;  // dist = dbase - kc
       if constexpr (kTable) {
         // element e at dist = dbase - kc: a constant offset from one base
-        int j0 = kBiasTop - dbase;  // table index of the lane's key 0
+        int j0 = tab_top - dbase;  // table index of the lane's key 0
         asm("" : "+v"(j0));          // one base address, the keys as read offsets
-        const float* tb = bias_lds + j0;
+        const float* tb = bias_lds + (kPack ? hq[qb] * tab_pitch : 0) + j0;
 #pragma unroll
         for (int e = 0; e < 16; ++e) bias[e] = tb[32 * blk + e];
       } else if constexpr (kProj) {
         proj_bias(kb, blk, bias);
       } else {
-        const int rel_row = qi[qb] * (int)p.rel_st;  // element offset of the row
+        const int rel_row = rel_row_of(qb);
         if constexpr (kTokEarly)
           tok_finish(rel_row, dbase - 32 * blk, row_ok[qb], traw[qb][blk], bias);
         else
@@ -873,7 +866,8 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
           for (int qb = 0; qb < kNqb; ++qb) {
             const int dbase = qi[qb] + delta - kb - 16 * half;  // dist = dbase - kc
-            int j0 = min(max(kBiasTop - dbase, 0), kBiasLdsFloats - kBlockK);
+            int j0 = min(max(tab_top - dbase, 0), tab_len - kBlockK);
+            if constexpr (kPack) j0 += hq[qb] * tab_pitch;
             asm("" : "+v"(j0));  // one base address, the keys as read offsets
             const float* tb = bias_lds + j0;
 #pragma unroll
@@ -896,7 +890,7 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
             bool done = false;
             if constexpr (kTokEarly) {
               const int dtop = qi[qb] + delta - kb - 16 * half - 32 * blk;
-              done = tok_dot(qi[qb] * (int)p.rel_st, dtop, traw[qb][blk], s[qb][blk]);
+              done = tok_dot(rel_row_of(qb), dtop, traw[qb][blk], s[qb][blk]);
             }
             if (done) {
               if (need_mask) {
@@ -1174,23 +1168,28 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
   // The bias table (shared-table layout) is read with the Q fragments and the
   // first tile; one wait for all three, then it goes to LDS.  The first tile's
   // barrier publishes it.
-  constexpr int kBiasPer = (2 * kBiasPad + kBiasLdsMax + kThreads - 1) / kThreads;
-  float tab[kBiasPer];
+  constexpr int kBiasPer = (kBiasLdsFloats + kThreads - 1) / kThreads;
+  float tab[kTable ? kBiasPer : 1];
   if (bias_in_lds) {
 #pragma unroll
     for (int i = 0; i < kBiasPer; ++i) {
       const int idx = tid + i * kThreads;  // table index
-      const int dist = kBiasTop - idx;
-      const uint32_t off = (uint32_t)dist < (uint32_t)rext ? (uint32_t)dist * Rel::kBytes
-                                                            : kOutOfRange;
-      tab[i] = Rel::load(rrel, off);
+      const int h = kPack ? idx / tab_pitch : 0;
+      const int dist = tab_top - (idx - h * tab_pitch);
+      const uint32_t off = (uint32_t)dist < (uint32_t)rext && h < pack
+                               ? (uint32_t)(dist + h * (int)p.rel_sh) * Rel::kBytes
+                               : kOutOfRange;
+      if (!kPack || i * kThreads < pack * tab_pitch) tab[i] = Rel::load(rrel, off);
     }
   }
   // Fused projection: this lane's row of r (channels 8 * half .. +7) as the B
   // operand, and the first tile's W^T rows.
   if constexpr (kProj) {
     float rv[8];
-    const uint32_t roff = (uint32_t)((qa + col) * (int)p.rel_st + 8 * half) * Rel::kBytes;
+    const uint32_t roff =
+        !kPack || row_ok[0]
+            ? (uint32_t)(qi[0] * (int)p.rel_st + hq[0] * (int)p.rel_sh + 8 * half) * Rel::kBytes
+            : kOutOfRange;
 #pragma unroll
     for (int c = 0; c < 8; ++c) rv[c] = Rel::load(rrel, roff + c * Rel::kBytes);
     split_bf16x8(rv, r_hi, r_lo);
@@ -1202,7 +1201,8 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
     for (int i = 0; i < kBiasPer; ++i) {
       const int idx = tid + i * kThreads;
-      if (idx < 2 * kBiasPad + kBiasLdsMax) bias_lds[idx] = tab[i];
+      if (idx < (kPack ? min(pack * tab_pitch, kBiasLdsFloats) : kBiasLdsFloats))
+        bias_lds[idx] = tab[i];
     }
     __builtin_amdgcn_s_waitcnt(kLgkm0);
   }
@@ -1220,11 +1220,14 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
   for (int qb = 0; qb < kNqb; ++qb) {
     const float l_tot = add_xor32(l_run[qb]);
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-    const int qi_e = qa + 32 * qb + (lane_e & 31);
-    const bool ok_e = qi_e < lq;
-    if (ok_e && nch > 1) {
+    const int r_e = row0 + 32 * qb + (lane_e & 31);
+    const int ql_e = kPack ? packed_query(p, r_e) : r_e;
+    const int qi_e = q0 + ql_e;
+    const int head_e = kPack ? head + r_e - ql_e * pack : head;
+    const bool ok_e = qi_e < it.q_end;
+if (ok_e && it.part >= 0) {
       // normalised O of the chunk (fp32) and its LSE in log2 units
-      const int64_t prow = ((int64_t)chunk * p.n_heads + head) * p.total_q + qs + qi_e;
+      const int64_t prow = ((int64_t)it.part * p.n_heads + head_e) * p.total_q + qs + qi_e;
       float* pbase = p.part_o + prow * D;
 #pragma unroll
       for (int db = 0; db < kDBlocks; ++db)
@@ -1236,7 +1239,7 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
       if (half_e == 0) p.part_lse[prow] = l_tot > 0.f ? m_run[qb] + __log2f(l_tot) : -INFINITY;
     } else if (ok_e) {
       uint16_t* obase = static_cast<uint16_t*>(p.out) + (int64_t)(qs + qi_e) * p.o_st +
-                        (int64_t)head * p.o_sh;
+                        (int64_t)head_e * p.o_sh;
 #pragma unroll
       for (int db = 0; db < kDBlocks; ++db) {
 #pragma unroll
@@ -1249,121 +1252,209 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
       }
       if (p.lse != nullptr && half_e == 0) {
         const float lse = l_tot > 0.f ? (m_run[qb] + __log2f(l_tot)) * kLn2 : -INFINITY;
-        p.lse[(int64_t)head * p.lse_sh + qs + qi_e] = lse;
+        p.lse[(int64_t)head_e * p.lse_sh + qs + qi_e] = lse;
       }
     }
   }
 }
 
-// Merge of split-KV partials (second pass after a split launch): kMergeParts
-// workgroups per (q tile, head, sequence), each an eighth of the tile's rows
-// (against a quarter: 1.3% faster on one sequence of 4096 over 4 heads, 3% at
-// 2048, within 1% elsewhere; sixteenths no better); a
-// tile whose range did not split was written by the prefill kernel itself and
-// is skipped.  32 threads share a row (head_dim / 32 consecutive d values each)
-// and a thread holds kRows rows; chunks go in rounds of kChunkBatch whose loads
-// (rows x chunks) are all in flight at once, merged online (running max over
-// the chunks' LSEs).
-constexpr int kMergeThreads = IFA4_MERGE_THREADS;
-constexpr int kMergeParts = IFA4_MERGE_PARTS;
-template <typename Sh, int D, typename Tag>
+template <typename Sh, int D, typename Tag, typename Rel, bool kProj, bool kTab, bool kPack>
+__global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
+    Sh::kWavesPerSimd, Sh::kWavesPerSimd))) void prefill_fwd_kernel(PrefillParams p) {
+  const int q_step = kPack ? p.q_step : Sh::kBlockQ;  // queries per tile
+  // ---- which (q tile, KV chunk, head, sequence): heaviest (last) q tiles first --
+  // A q tile's chunks (split KV; one when not splitting) are consecutive, so
+  // a chunk that ends early is followed by the next q tile's work.
+  int qtile, chunk, head, seq;
+  if (p.xcd_spread) {  // ragged (prefill_order)
+    const int x = blockIdx.x & 7;
+    int slot = blockIdx.x >> 3;
+    const int m = slot % p.xcd_unit;
+    slot /= p.xcd_unit;
+    const int k = slot % p.xcd_heads;
+    slot /= p.xcd_heads;
+    const int rounds = (p.batch + p.xcd_spread - 1) / p.xcd_spread;
+    const int qc = slot / rounds;
+    seq = (slot + qc) % rounds * p.xcd_spread + ((x + 7 * qc) & (p.xcd_spread - 1));
+    if (seq >= p.batch) return;
+    head = (p.xcd_spread > 1 ? x / p.xcd_spread : x * p.xcd_heads + k) * p.xcd_unit + m;
+    qtile = p.n_qtiles - 1 - qc / p.n_chunks;
+    chunk = qc % p.n_chunks;
+  } else if (p.xcd_pairs) {
+    // Workgroup i runs on XCD i % 8.  Give XCD x the (sequence, kv head) pairs
+    // x, x+8, ... so their K/V stay in that XCD's L2; heaviest q tiles first.
+    const int x = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const int per_xcd = p.xcd_pairs;  // pairs per XCD
+    const int per_tile = per_xcd * p.tile_group;
+    const int qc = slot / per_tile;
+    qtile = p.n_qtiles - 1 - qc / p.n_chunks;
+    chunk = qc % p.n_chunks;
+    const int rem = slot % per_tile;
+    const int pair = x + 8 * (rem / p.tile_group);
+    const int kv_heads = p.tile_heads / p.tile_group;
+    seq = pair / kv_heads;
+    head = (pair % kv_heads) * p.tile_group + rem % p.tile_group;
+  } else {
+    const int per_tile = p.tile_heads * p.batch;
+    const int lin = blockIdx.x;
+    const int qc = lin / per_tile;
+    qtile = p.n_qtiles - 1 - qc / p.n_chunks;
+    chunk = qc % p.n_chunks;
+    const int rem = lin % per_tile;
+    head = rem % p.tile_heads;
+    seq = rem / p.tile_heads;
+    if (p.ragged) seq = (seq + qc) % p.batch;
+  }
+
+  WorkItem it;
+  set_sequence(p, it, seq);
+  it.q0 = qtile * q_step;
+  if (it.q0 >= it.lq) return;
+  it.q_end = min(it.q0 + q_step, it.lq);
+  it.kvh = head / p.tile_group;
+  it.head0 = kPack ? head * p.pack : head;
+  // key range of the workgroup (tile pruning, then this KV chunk)
+  const TileRange tr = tile_range<Sh>(p, it.q0, it.q_end, it.lk, it.qpos);
+  const int nch = tile_chunks(p, tr);
+  if (chunk >= nch) return;
+  it.kt_beg = tr.beg;
+  it.kt_end = tr.end;
+  it.part = -1;
+  if (nch > 1) {
+    const int c0 = (tr.beg / p.chunk_tiles + chunk) * p.chunk_tiles;
+    it.kt_beg = max(tr.beg, c0);
+    it.kt_end = min(tr.end, c0 + p.chunk_tiles);
+    it.part = chunk;
+  }
+  prefill_work<Sh, D, Tag, Rel, kProj, kTab, kPack>(p, it);
+}
+
+// Merge of split-KV partials (second pass after a split launch).  32 threads
+// share a row (head_dim / 32 consecutive d values each), a workgroup's 8 such
+// teams are 8 / GROUPS rows x GROUPS groups of chunks: group g merges the chunks
+// whose absolute index is g modulo GROUPS, up to kChunkBatch of them loaded at
+// once, online (running max over their LSEs), and the groups of a row meet in
+// LDS.  A row of n chunks so takes n / (4 GROUPS) dependent memory rounds; the
+// host picks GROUPS by the rows and chunk slots of the call.  A query tile
+// whose range did not split was written by the prefill kernel and is skipped.
+// Chunks go to groups and rounds by absolute index, so the chunks meet in the
+// same order whatever the pruning: chunks a pruned range drops hold no key (LSE
+// -inf) and leave the running sums bit-unchanged.
+constexpr int kMergeThreads = 256;
+template <typename Sh, int D, typename Tag, int GROUPS>
 __global__ __launch_bounds__(kMergeThreads) void prefill_merge_kernel(PrefillParams p) {
   using E = Elem<Tag>;
-  constexpr int kTpr = 32;                          // threads per row
-  constexpr int kPer = D / kTpr;                    // d values per thread
-  constexpr int kStride = kMergeThreads / kTpr;     // rows per pass of the workgroup
-  constexpr int kRows = Sh::kBlockQ / kMergeParts / kStride;  // rows per thread
-  static_assert(kRows >= 1 && kRows * kStride * kMergeParts == Sh::kBlockQ,
-                "merge workgroups cover the query tile's rows exactly");
-  const int qtile = blockIdx.x / kMergeParts, part = blockIdx.x % kMergeParts;
+  constexpr int kTpr = 32;                         // threads per row
+  constexpr int kPer = D / kTpr;                   // d values per thread
+  constexpr int kRows = kMergeThreads / kTpr / GROUPS;  // rows per workgroup
+  constexpr int kChunkBatch = IFA4_MERGE_BATCH;
+  const int team = (int)threadIdx.x / kTpr;
   const int head = blockIdx.y, seq = blockIdx.z;
   const SeqBounds bq = seq_bounds(p.cu_q, seq, p.total_q);
   const SeqBounds bk = seq_bounds(p.cu_k, seq, p.total_k);
-  const int q0 = qtile * Sh::kBlockQ;
-  if (q0 >= bq.len) return;
+  const int row = blockIdx.x * kRows + team / GROUPS, grp = team % GROUPS;
+  const int q0 = row / p.q_step * p.q_step;
+  const int q_end = min(q0 + p.q_step, bq.len);
   const int qpos = p.bottom_right ? bk.len - bq.len : 0;
-  const TileRange tr = tile_range<Sh>(p, q0, bq.len, bk.len, qpos);
+  const TileRange tr = tile_range<Sh>(p, q0, q_end, bk.len, qpos);
   const int nch = tile_chunks(p, tr);
-  if (nch <= 1) return;
-  const int r0 = q0 + part * (Sh::kBlockQ / kMergeParts) + (int)threadIdx.x / kTpr;
+  const bool live = row < q_end && nch > 1;
+  if (GROUPS == 1 && !live) return;
   const int d0 = ((int)threadIdx.x % kTpr) * kPer;
   const int64_t chunk_rows = (int64_t)p.n_heads * p.total_q;
-  const int64_t row0 = (int64_t)head * p.total_q + bq.start;
-  float m[kRows], l[kRows], acc[kRows][kPer];
+  const int64_t row0 = (int64_t)head * p.total_q + bq.start + row;
+  float m = -INFINITY, l = 0.f;
+  float acc[kPer];
 #pragma unroll
-  for (int i = 0; i < kRows; ++i) {
-    m[i] = -INFINITY;
-    l[i] = 0.f;
+  for (int e = 0; e < kPer; ++e) acc[e] = 0.f;
+  if (live) {
+    // slot c of this query tile is absolute chunk tr.beg / chunk_tiles + c
+    constexpr int kRound = kChunkBatch * GROUPS;
+    const int lead = (tr.beg / p.chunk_tiles) % kRound;
+    for (int c0 = grp - lead; c0 < nch; c0 += kRound) {
+      float ls[kChunkBatch];
+      float os[kChunkBatch][kPer];
 #pragma unroll
-    for (int e = 0; e < kPer; ++e) acc[i][e] = 0.f;
-  }
-  // kChunkBatch chunks per round: every load of a round (its rows x chunks)
-  // is issued before the first is used
-  constexpr int kChunkBatch = IFA4_MERGE_BATCH;
-  // Rounds start at absolute chunk indices that are multiples of kChunkBatch
-  // (slot k of this query tile is absolute chunk tr.beg / chunk_tiles + k), so
-  // the chunks meet in the same rounds whatever the pruning: chunks a pruned
-  // range drops hold no key (LSE -inf) and leave the running sums bit-unchanged.
-  const int lead = (tr.beg / p.chunk_tiles) % kChunkBatch;
-  for (int c0 = -lead; c0 < nch; c0 += kChunkBatch) {
-    float ls[kChunkBatch][kRows];
-    float os[kChunkBatch][kRows][kPer];
-#pragma unroll
-    for (int cb = 0; cb < kChunkBatch; ++cb) {
-#pragma unroll
-      for (int i = 0; i < kRows; ++i) {
-        const int row = r0 + kStride * i;
-        const bool ok = row < bq.len && c0 + cb >= 0 && c0 + cb < nch;
-        const int64_t prow = (ok ? c0 + cb : 0) * chunk_rows + row0 + row;
-        ls[cb][i] = ok ? p.part_lse[prow] : -INFINITY;
+      for (int cb = 0; cb < kChunkBatch; ++cb) {
+        const int c = c0 + cb * GROUPS;
+        const bool ok = c >= 0 && c < nch;
+        const int64_t prow = (ok ? c : 0) * chunk_rows + row0;
+        ls[cb] = ok ? p.part_lse[prow] : -INFINITY;
         if constexpr (kPer == 4) {
           const f32x4_t v =
               ok ? *reinterpret_cast<const f32x4_t*>(p.part_o + prow * D + d0) : f32x4_t{};
 #pragma unroll
-          for (int e = 0; e < 4; ++e) os[cb][i][e] = v[e];
+          for (int e = 0; e < 4; ++e) os[cb][e] = v[e];
         } else {
 #pragma unroll
-          for (int e = 0; e < kPer; ++e) os[cb][i][e] = ok ? p.part_o[prow * D + d0 + e] : 0.f;
+          for (int e = 0; e < kPer; ++e) os[cb][e] = ok ? p.part_o[prow * D + d0 + e] : 0.f;
         }
       }
-    }
+      float mn = m;
 #pragma unroll
-    for (int i = 0; i < kRows; ++i) {
-      float mn = m[i];
-#pragma unroll
-      for (int cb = 0; cb < kChunkBatch; ++cb) mn = fmaxf(mn, ls[cb][i]);
+      for (int cb = 0; cb < kChunkBatch; ++cb) mn = fmaxf(mn, ls[cb]);
       const float mu = mn == -INFINITY ? 0.f : mn;
-      const float a_old = fast_exp2(m[i] - mu);
-      l[i] *= a_old;
+      const float a_old = fast_exp2(m - mu);
+      l *= a_old;
 #pragma unroll
-      for (int e = 0; e < kPer; ++e) acc[i][e] *= a_old;
+      for (int e = 0; e < kPer; ++e) acc[e] *= a_old;
 #pragma unroll
       for (int cb = 0; cb < kChunkBatch; ++cb) {
-        const float a_new = fast_exp2(ls[cb][i] - mu);
-        l[i] += a_new;
+        const float a_new = fast_exp2(ls[cb] - mu);
+        l += a_new;
 #pragma unroll
-        for (int e = 0; e < kPer; ++e) acc[i][e] += a_new * os[cb][i][e];
+        for (int e = 0; e < kPer; ++e) acc[e] += a_new * os[cb][e];
       }
-      m[i] = mn;
+      m = mn;
     }
   }
+  if constexpr (GROUPS > 1) {
+    __shared__ float part[kMergeThreads / kTpr][kTpr * kPer + 2];
 #pragma unroll
-  for (int i = 0; i < kRows; ++i) {
-    const int row = r0 + kStride * i;
-    if (row >= bq.len) continue;
-    const float inv = l[i] > 0.f ? 1.f / l[i] : 0.f;
-    uint16_t* dst = static_cast<uint16_t*>(p.out) + (int64_t)(bq.start + row) * p.o_st +
-                    (int64_t)head * p.o_sh + d0;
-    if constexpr (kPer == 4) {
-      *reinterpret_cast<u32x2_t*>(dst) = u32x2_t{E::pack2(acc[i][0] * inv, acc[i][1] * inv),
-                                                 E::pack2(acc[i][2] * inv, acc[i][3] * inv)};
-    } else {
-      *reinterpret_cast<uint32_t*>(dst) = E::pack2(acc[i][0] * inv, acc[i][1] * inv);
+    for (int e = 0; e < kPer; ++e) part[team][d0 + e] = acc[e];
+    if (d0 == 0) {
+      part[team][D] = m;
+      part[team][D + 1] = l;
     }
-    if (p.lse != nullptr && d0 == 0)
-      p.lse[(int64_t)head * p.lse_sh + bq.start + row] =
-          l[i] > 0.f ? (m[i] + __log2f(l[i])) * kLn2 : -INFINITY;
+    __syncthreads();
+    if (!live || grp != 0) return;
+    float mn = m;
+#pragma unroll
+    for (int g = 1; g < GROUPS; ++g) mn = fmaxf(mn, part[team + g][D]);
+    const float mu = mn == -INFINITY ? 0.f : mn;
+    const float a0 = fast_exp2(m - mu);
+    l *= a0;
+#pragma unroll
+    for (int e = 0; e < kPer; ++e) acc[e] *= a0;
+#pragma unroll
+    for (int g = 1; g < GROUPS; ++g) {
+      const float a = fast_exp2(part[team + g][D] - mu);
+      l += a * part[team + g][D + 1];
+#pragma unroll
+      for (int e = 0; e < kPer; ++e) acc[e] += a * part[team + g][d0 + e];
+    }
+    m = mn;
   }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  uint16_t* dst = static_cast<uint16_t*>(p.out) + (int64_t)(bq.start + row) * p.o_st +
+                  (int64_t)head * p.o_sh + d0;
+  if constexpr (kPer == 4) {
+    *reinterpret_cast<u32x2_t*>(dst) =
+        u32x2_t{E::pack2(acc[0] * inv, acc[1] * inv), E::pack2(acc[2] * inv, acc[3] * inv)};
+  } else {
+    *reinterpret_cast<uint32_t*>(dst) = E::pack2(acc[0] * inv, acc[1] * inv);
+  }
+  if (p.lse != nullptr && d0 == 0)
+    p.lse[(int64_t)head * p.lse_sh + bq.start + row] =
+        l > 0.f ? (m + __log2f(l)) * kLn2 : -INFINITY;
+}
+
+template <typename Sh, int D, typename Tag, int GROUPS>
+void launch_merge(const PrefillParams& p, hipStream_t stream) {
+  constexpr int kRows = kMergeThreads / 32 / GROUPS;
+  hipLaunchKernelGGL((prefill_merge_kernel<Sh, D, Tag, GROUPS>),
+                     dim3((p.max_q + kRows - 1) / kRows, p.n_heads, p.batch), dim3(kMergeThreads),
+                     0, stream, p);
 }
 
 // Workgroup order and grid of a call.  Pairs in fixed XCDs suit equal lengths
@@ -1382,14 +1473,14 @@ __global__ __launch_bounds__(kMergeThreads) void prefill_merge_kernel(PrefillPar
 // against 88), as with fewer sequences than XCDs to take turns on, and for the
 // KV chunks of a split call (3 x 333..512 tokens over 3K..9K keys: 65.3 against 69.0).
 int64_t prefill_order(PrefillParams& p) {
-  const int pairs = p.batch * (p.n_heads / p.group);
+  const int pairs = p.batch * (p.tile_heads / p.tile_group);
   const int64_t tiles = (int64_t)p.n_qtiles * p.n_chunks;
   p.xcd_spread = 0;
   p.xcd_pairs = pairs % 8 == 0 ? pairs / 8 : 0;
   if (p.ragged && p.n_chunks == 1) {
-    int unit = p.group < 4 ? p.group : 4;
-    while (p.group % unit != 0) --unit;
-    const int units = p.n_heads / unit;  // per sequence
+    int unit = p.tile_group < 4 ? p.tile_group : 4;
+    while (p.tile_group % unit != 0) --unit;
+    const int units = p.tile_heads / unit;  // per sequence
     const int spread = units % 8 == 0 ? 1 : 8 % units == 0 ? 8 / units : 0;
     if (unit > 1 && spread > 0 && p.batch >= spread) {
       p.xcd_unit = unit;
@@ -1399,51 +1490,56 @@ int64_t prefill_order(PrefillParams& p) {
     }
     p.xcd_pairs = 0;
   }
-  return tiles * p.n_heads * p.batch;
+  return tiles * p.tile_heads * p.batch;
 }
 
-template <typename Sh, int D, typename Tag, typename Rel, bool kProj, bool kTab = false>
+template <typename Sh, int D, typename Tag, typename Rel, bool kProj, bool kTab, bool kPack>
 hipError_t launch_prefill_t(const PrefillParams& p_in, hipStream_t stream) {
   PrefillParams p = p_in;
   if (p.n_chunks < 1) p.n_chunks = 1;
   const int64_t blocks = prefill_order(p);
   if (blocks <= 0) return hipSuccess;
-  hipLaunchKernelGGL((prefill_fwd_kernel<Sh, D, Tag, Rel, kProj, kTab>), dim3((unsigned)blocks),
+  hipLaunchKernelGGL((prefill_fwd_kernel<Sh, D, Tag, Rel, kProj, kTab, kPack>), dim3((unsigned)blocks),
                      dim3(Sh::kThreads), 0, stream, p);
   if constexpr (!kProj) {  // the fused projection never splits
     if (p.chunk_tiles > 0) {
       const hipError_t e = hipGetLastError();
       if (e != hipSuccess) return e;
-      hipLaunchKernelGGL((prefill_merge_kernel<Sh, D, Tag>),
-                         dim3(p.n_qtiles * kMergeParts, p.n_heads, p.batch), dim3(kMergeThreads),
-                         0, stream, p);
+      // Groups pay where a call has few rows of many chunks: the rounds of a row
+      // are then all the merge waits for.  With many rows more workgroups cost
+      // more.  Whole calls, 1 / 2 / 8 groups (one box, us): 32 rows x up to 32
+      // chunks 19.3 / 17.2 / 15.5, 720 x 36 28.7 / 27.6 / 26.9, 1.8K x 36 32.5 / 31.5 /
+      // 31.2, 2K x 4 13.0 / 13.4 / 14.4, 9.3K x 6 63.8 / 65.8 / 71.5.
+      if (p.seen_chunks > 8 && (int64_t)p.n_heads * p.total_q <= 2048)
+        launch_merge<Sh, D, Tag, 8>(p, stream);
+      else
+        launch_merge<Sh, D, Tag, 1>(p, stream);
     }
   }
   return hipGetLastError();
 }
 
+template <int D, typename Tag, bool kTab, bool kPack>
+hipError_t launch_prefill_bias(const PrefillParams& p, hipStream_t stream) {
+  switch (p.rel_dtype) {
+    case 0: return launch_prefill_t<Shape, D, Tag, RelBf16, false, kTab, kPack>(p, stream);
+    case 1: return launch_prefill_t<Shape, D, Tag, RelF16, false, kTab, kPack>(p, stream);
+    default: return launch_prefill_t<Shape, D, Tag, RelF32, false, kTab, kPack>(p, stream);
+  }
+}
+
 template <int D, typename Tag>
 hipError_t launch_prefill_rel(const PrefillParams& p, hipStream_t stream) {
   if (p.wt != nullptr) {  // fused projection: r in bf16 or fp32
-    return p.rel_dtype == 2 ? launch_prefill_t<ProjShape, D, Tag, RelF32, true>(p, stream)
-                            : launch_prefill_t<ProjShape, D, Tag, RelBf16, true>(p, stream);
+    return p.rel_dtype == 2
+               ? launch_prefill_t<ProjShape, D, Tag, RelF32, true, false, false>(p, stream)
+               : launch_prefill_t<ProjShape, D, Tag, RelBf16, true, false, false>(p, stream);
   }
-  // one per-head table shared by every token (token stride 0), short enough
-  // for LDS: the table instantiation; per-token rows (or no bias): the other
-  const bool tab =
-      IFA4_BIAS_LDS && p.rel_st == 0 && p.rel_extent > 0 && p.rel_extent <= kBiasLdsMax;
-  if (tab) {
-    switch (p.rel_dtype) {
-      case 0: return launch_prefill_t<Shape, D, Tag, RelBf16, false, true>(p, stream);
-      case 1: return launch_prefill_t<Shape, D, Tag, RelF16, false, true>(p, stream);
-      default: return launch_prefill_t<Shape, D, Tag, RelF32, false, true>(p, stream);
-    }
-  }
-  switch (p.rel_dtype) {
-    case 0: return launch_prefill_t<Shape, D, Tag, RelBf16, false>(p, stream);
-    case 1: return launch_prefill_t<Shape, D, Tag, RelF16, false>(p, stream);
-    default: return launch_prefill_t<Shape, D, Tag, RelF32, false>(p, stream);
-  }
+  if (prefill_tab(p))
+    return p.pack > 1 ? launch_prefill_bias<D, Tag, true, true>(p, stream)
+                      : launch_prefill_bias<D, Tag, true, false>(p, stream);
+  return p.pack > 1 ? launch_prefill_bias<D, Tag, false, true>(p, stream)
+                    : launch_prefill_bias<D, Tag, false, false>(p, stream);
 }
 
 }  // namespace
@@ -1451,6 +1547,12 @@ hipError_t launch_prefill_rel(const PrefillParams& p, hipStream_t stream) {
 int prefill_block_q() { return Shape::kBlockQ; }
 int prefill_proj_block_q() { return ProjShape::kBlockQ; }
 int prefill_block_k() { return Shape::kBlockK; }
+bool prefill_tab_packs(int rel_extent, int pack) {
+  return pack * bias_pack_pitch(rel_extent, pack, Shape::kBiasPad) <= kBiasPackFloats;
+}
+bool prefill_tab(const PrefillParams& p) {
+  return IFA4_BIAS_LDS && p.rel_st == 0 && p.rel_extent > 0 && p.rel_extent <= kBiasLdsMax;
+}
 int prefill_waves() { return Shape::kWaves; }
 
 hipError_t launch_prefill(const PrefillParams& p, int head_dim, int qkv_dtype,

@@ -205,9 +205,26 @@ constexpr int64_t kPrefillChunkPct = IFA4_PREFILL_CHUNK_PCT;
 #endif
 constexpr int64_t kPrefillSplitWideMinTiles = 16;
 
+// Packed rows: the query heads of a kv head share query tiles (block_q / group
+// queries x group heads) when every sequence fits one tile of block_q queries and
+// packing leaves at most three quarters of the tiles.  A sequence of a few
+// queries otherwise takes one workgroup per head with one or two of its four
+// waves at work, each streaming the same K/V.  With it against without (one box,
+// us, Hq 8 / Hkv 2, d 128): 12 x 2..5 queries over 1K..8K keys 42.4 -> 22.9, 24 x
+// 2..8 91.6 -> 41.3, Hq 8 / Hkv 1 56.5 -> 24.6, 3 x 20..40 over 3K..9K 26.8 -> 22.4,
+// x 50..96 31.3 -> 29.2.  Past a tile per head it no longer pays on every call:
+// 3 x 120..200 45 -> 39, but 333..410 64 -> 69, 16 x 17..300 without a cache
+// 15.5 -> 18.8 (fewer, fuller workgroups leave CUs idle).
+inline bool prefill_packs(int64_t group, int64_t max_q, int64_t block_q) {
+  if (group <= 1 || group > block_q || max_q <= 0 || max_q > block_q) return false;
+  const int64_t step = block_q / group;
+  return 4 * ((max_q + step - 1) / step) <= 3 * group;
+}
+
 struct PrefillSplit {
   int32_t chunk_tiles;  // 0: no split
   int32_t n_chunks;     // chunk slots per query tile in the grid
+  int32_t seen_chunks;  // of them, those a query tile with pruned tiles can need
 };
 
 // Masks of a call: a sequence's query 0 sits at key position qpos.
@@ -264,7 +281,7 @@ inline PrefillSplit prefill_split_for(int64_t batch, int64_t n_heads, int64_t ma
                                       int64_t max_k, bool causal, int64_t window_left,
                                       bool bottom_right, bool no_prune, int32_t block_q,
                                       int32_t block_k, int32_t forced_chunk) {
-  PrefillSplit s{0, 1};
+  PrefillSplit s{0, 1, 1};
   if (batch <= 0 || max_q <= 0 || max_k <= 0) return s;
   const PrefillMasks masks{causal && !(bottom_right && window_left < 0), window_left,
                            bottom_right && max_k > max_q ? max_k - max_q : int64_t(0)};
@@ -312,12 +329,14 @@ inline PrefillSplit prefill_split_for(int64_t batch, int64_t n_heads, int64_t ma
   const int64_t key_tiles = (max_k + block_k - 1) / block_k;
   s.chunk_tiles = (int32_t)chunk;
   s.n_chunks = (int32_t)((key_tiles + chunk - 1) / chunk);
-  if (causal && window_left >= 0 && !no_prune) {
+  if (s.n_chunks < 1) s.n_chunks = 1;
+  s.seen_chunks = s.n_chunks;
+  if (causal && window_left >= 0) {
     const int64_t span = (block_q + window_left + block_k - 1) / block_k + 1;  // tiles
     const int64_t slots = (span + chunk - 1) / chunk + 1;
-    if (slots < s.n_chunks) s.n_chunks = (int32_t)slots;
+    if (slots < s.n_chunks) s.seen_chunks = (int32_t)slots;
+    if (!no_prune) s.n_chunks = s.seen_chunks;
   }
-  if (s.n_chunks < 1) s.n_chunks = 1;
   return s;
 }
 

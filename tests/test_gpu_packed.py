@@ -1,0 +1,91 @@
+"""Prefill calls of a few queries per sequence over a cache: packed rows (the
+query heads of a kv head share query tiles) and the merge of many chunks.
+
+Packed rows start at 96 queries for groups of four (three quarters of the tiles);
+sizes sit on both sides of that, at tile edges and with groups that do not divide
+the 128 rows (3, 6, 12).  Everything is compared with the fp32 oracle (16-bit
+rounding of P and of the output: 2e-2; fp32 LSE: 1e-3), and pruned with unpruned
+launches bit for bit.
+"""
+import pytest
+import torch
+
+from inkling_fa4 import _abi, inkling_fa4_rel_attention, testing
+from oracle import ref_rel_attn_with_lse
+
+
+def _run(c, flags=0, bottom_right=True):
+    return inkling_fa4_rel_attention(*c.args(), causal=c.causal, window_size=c.window_size,
+                                     softmax_scale=c.scale, return_lse=True,
+                                     bottom_right=bottom_right, _flags=flags)
+
+
+def _check(case, dev, bottom_right=True):
+    print(f"{case.name}: q {tuple(case.q.shape)}, k {tuple(case.k.shape)}, causal {case.causal}, "
+          f"window {case.window_left}, bottom-right {bottom_right}", flush=True)
+    c = case.to(dev)
+    out, lse = _run(c, 0, bottom_right)
+    want_out, want_lse = ref_rel_attn_with_lse(
+        case.q, case.k, case.v, case.rel, case.cu_q, case.cu_k, case.scale, case.rel_extent,
+        causal=case.causal, window_left=case.window_or_none, bottom_right=bottom_right)
+    rows = ~torch.isnan(want_out).any(-1)  # rows with a visible key
+    out, lse = out.cpu(), lse.cpu()
+    torch.testing.assert_close(out.float()[rows], want_out.float()[rows], atol=2e-2, rtol=2e-2)
+    torch.testing.assert_close(lse.T[rows], want_lse.T[rows], atol=1e-3, rtol=0)
+    assert bool((out[~rows] == 0).all()) and bool((lse.T[~rows] == float("-inf")).all())
+    full = _run(c, _abi.IFA4_FLAG_NO_PRUNE, bottom_right)
+    assert torch.equal(full[0].cpu(), out) and torch.equal(full[1].cpu(), lse)
+    two, lse2 = _run(c, _abi.IFA4_FLAG_SPLIT_KV_2, bottom_right)
+    torch.testing.assert_close(lse2.cpu(), lse, atol=1e-4, rtol=0)
+    torch.testing.assert_close(two.float().cpu(), out.float(), atol=2e-2, rtol=2e-2)
+
+
+# (hq, hkv, longest query length): groups 2, 3, 4, 6, 8, 12, 16, 64; the last two
+# lengths of each are the edge of the rule and just past it
+@pytest.mark.gpu
+@pytest.mark.parametrize("hq,hkv,top", [(4, 2, 64), (4, 2, 65), (6, 2, 84), (8, 2, 5), (8, 2, 96),
+                                        (8, 2, 97), (12, 2, 63), (16, 2, 33), (24, 2, 8),
+                                        (16, 1, 96), (64, 1, 3)])
+def test_packed_groups_and_lengths(cuda, hq, hkv, top):
+    lens_q = [1, top, max(1, top - 1), 2, 0]
+    lens_k = [70, 700 + top, 1500, 2, 300]
+    case = testing.make_case("packed", lens_q, lens_k, hq, hkv, 128, torch.bfloat16,
+                             seed=10 * hq + top, rel_table=False, rel_extent=200,
+                             rel_dtype=torch.bfloat16, scale=0.1)
+    _check(case, cuda)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("head_dim,dtype", [(128, torch.bfloat16), (64, torch.float16)])
+@pytest.mark.parametrize("rel_table,extent,rel_dtype", [(True, 128, torch.float32),
+                                                        (True, 1024, torch.bfloat16),
+                                                        (False, 300, torch.float16),
+                                                        (False, 129, torch.float32)])
+def test_packed_bias_forms(cuda, head_dim, dtype, rel_table, extent, rel_dtype):
+    # a shared table of 1024 is too long for the packed tables' LDS: unpacked
+    case = testing.make_case("packed_bias", [7, 31, 2], [900, 40, 1300], 8, 2, head_dim, dtype,
+                             seed=extent, rel_table=rel_table, rel_extent=extent,
+                             rel_width=extent + 3, rel_dtype=rel_dtype, scale=0.1)
+    _check(case, cuda)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("causal,window,bottom_right", [(False, -1, True), (True, -1, False),
+                                                        (False, 50, False), (True, 0, True),
+                                                        (True, 63, True), (True, 200, True)])
+def test_packed_masks(cuda, causal, window, bottom_right):
+    # sequence 1 has more queries than keys: rows without a visible key bottom-right
+    case = testing.make_case("packed_mask", [5, 60, 17], [640, 40, 2100], 8, 2, 128,
+                             torch.bfloat16, seed=31, causal=causal, window_left=window,
+                             scale=0.15)
+    _check(case, cuda, bottom_right)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("keys", [1300, 9000])
+def test_merge_of_many_chunks(cuda, head_dim, keys):
+    # few rows over tens of chunks: eight groups of chunks per row
+    case = testing.make_case("many_chunks", [3, 20], [keys, keys // 3], 4, 4, head_dim,
+                             torch.bfloat16, seed=keys, scale=0.1)
+    _check(case, cuda)
