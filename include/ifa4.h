@@ -186,8 +186,16 @@ size_t ifa4_prefill_workspace_bytes(const ifa4_args* args);
 int32_t ifa4_prefill_fwd_ws(const ifa4_args* args, void* workspace, size_t workspace_bytes,
                             void* stream);
 
-/* Prefill with the fused relative-logit projection (ifa4_rel_proj). */
+/*
+ * Prefill with the fused relative-logit projection (ifa4_rel_proj).  The _ws form
+ * splits the KV range of underfilled grids in a workspace as ifa4_prefill_fwd_ws
+ * does (same rules for the workspace; ifa4_prefill_rproj_workspace_bytes is 0 for
+ * a call that does not split); results equal up to the rounding of the merge.
+ */
 int32_t ifa4_prefill_rproj_fwd(const ifa4_args* args, const ifa4_rel_proj* proj, void* stream);
+size_t ifa4_prefill_rproj_workspace_bytes(const ifa4_args* args, const ifa4_rel_proj* proj);
+int32_t ifa4_prefill_rproj_fwd_ws(const ifa4_args* args, const ifa4_rel_proj* proj,
+                                  void* workspace, size_t workspace_bytes, void* stream);
 
 /* Tile shape ifa4_prefill_fwd uses for these arguments, and the KV split of
  * ifa4_prefill_fwd_ws (kv_chunk). */

@@ -212,13 +212,15 @@ int prefill_pack(const ifa4_args* a) {
   return (int)group;
 }
 
-ifa4::PrefillSplit prefill_split(const ifa4_args* a, int pack) {
+ifa4::PrefillSplit prefill_split(const ifa4_args* a, int pack, bool proj = false) {
   return ifa4::prefill_split_for(a->batch, a->n_heads / pack, a->max_seqlen_q, a->max_seqlen_k,
                                  a->causal != 0, a->window_left,
                                  (a->flags & IFA4_FLAG_BOTTOM_RIGHT) != 0,
                                  (a->flags & IFA4_FLAG_NO_PRUNE) != 0,
-                                 ifa4::prefill_block_q() / pack, ifa4::prefill_block_k(),
-                                 (a->flags & IFA4_FLAG_SPLIT_KV_2) ? 2 : 0);
+                                 (proj ? ifa4::prefill_proj_block_q() : ifa4::prefill_block_q()) / pack,
+                                 ifa4::prefill_block_k(),
+                                 (a->flags & IFA4_FLAG_SPLIT_KV_2) ? 2 : 0,
+                                 proj ? ifa4::kProjSplitRule : ifa4::kPrefillSplitRule);
 }
 
 // Split-KV plan of a prefill call and the workspace it needs: partial O
@@ -229,14 +231,79 @@ struct PrefillWorkspace {
   int64_t o_bytes, lse_bytes;
   int64_t total() const { return split.chunk_tiles > 0 ? o_bytes + lse_bytes : 0; }
 };
-PrefillWorkspace prefill_workspace(const ifa4_args* a) {
+PrefillWorkspace prefill_workspace(const ifa4_args* a, bool proj = false) {
   PrefillWorkspace w;
-  w.pack = prefill_pack(a);
-  w.split = prefill_split(a, w.pack);
+  w.pack = proj ? 1 : prefill_pack(a);
+  w.split = prefill_split(a, w.pack, proj);
   const int64_t rows = (int64_t)w.split.n_chunks * a->n_heads * a->total_q;
   w.o_bytes = (rows * a->head_dim * 4 + 255) / 256 * 256;
   w.lse_bytes = (rows * 4 + 255) / 256 * 256;
   return w;
+}
+
+// The split of a call in its workspace; false when that is missing or too small.
+bool set_split(ifa4::PrefillParams& p, const PrefillWorkspace& w, void* workspace,
+               size_t workspace_bytes) {
+  if (w.total() == 0) return true;
+  if (workspace == nullptr || workspace_bytes < (size_t)w.total() || !aligned(workspace, 256))
+    return false;
+  p.chunk_tiles = w.split.chunk_tiles;
+  p.n_chunks = w.split.n_chunks;
+  p.seen_chunks = w.split.seen_chunks;
+  p.part_o = static_cast<float*>(workspace);
+  p.part_lse = reinterpret_cast<float*>(static_cast<char*>(workspace) + w.o_bytes);
+  return true;
+}
+
+// Checks of a fused-projection call; *out: the arguments with r in the place of rel.
+int32_t check_rproj(const ifa4_args* args, const ifa4_rel_proj* pr, ifa4_args* out) {
+  if (args == nullptr || pr == nullptr || pr->struct_size != sizeof(ifa4_rel_proj))
+    return IFA4_EINVAL;
+  if (pr->d_rel != 16) return IFA4_EUNSUPPORTED;
+  if (args->rel_dtype != IFA4_BF16 && args->rel_dtype != IFA4_FP32) return IFA4_EUNSUPPORTED;
+  if (pr->r_stride_t < 0 || pr->r_stride_h < 0) return IFA4_EINVAL;
+  // The rel arguments of ifa4_args describe r here: checked below, not by check_args.
+  ifa4_args& b = *out;
+  b = *args;
+  b.rel = pr->r;
+  b.rel_stride_t = 0;
+  b.rel_stride_h = 0;
+  const int32_t st = check_args(&b);
+  if (st != IFA4_OK) return st;
+  if (args->batch == 0 || args->max_seqlen_q == 0) return IFA4_OK;
+  if (args->rel_extent > 0) {
+    const int64_t esize = args->rel_dtype == IFA4_FP32 ? 4 : 2;
+    if (pr->r == nullptr || pr->wt == nullptr || !aligned(pr->r, esize) || !aligned(pr->wt, 16))
+      return IFA4_EINVAL;
+    if (pr->r_stride_t != 0 && pr->r_stride_t < 16) return IFA4_EUNSUPPORTED;
+    if (((int64_t)args->max_seqlen_q + ifa4::prefill_proj_block_q()) * pr->r_stride_t * esize >=
+            (int64_t(1) << 31) ||
+        (int64_t)args->rel_width * 64 >= (int64_t(1) << 31))
+      return IFA4_EUNSUPPORTED;
+  }
+  return IFA4_OK;
+}
+
+// split: in the caller's workspace, when the tile table asks for one.
+int32_t run_rproj(const ifa4_args* args, const ifa4_rel_proj* pr, bool split, void* workspace,
+                  size_t workspace_bytes, void* stream) {
+  ifa4_args b;
+  const int32_t st = check_rproj(args, pr, &b);
+  if (st != IFA4_OK) return st;
+  if (args->batch == 0 || args->max_seqlen_q == 0) return IFA4_OK;
+  ifa4::PrefillParams p = make_prefill_params(&b);
+  p.rel = pr->r;
+  p.rel_st = pr->r_stride_t;
+  p.rel_sh = pr->r_stride_h;
+  p.wt = args->rel_extent > 0 ? pr->wt : nullptr;  // no bias at all: the plain kernel
+  if (p.wt != nullptr) {
+    set_tiles(p, args, ifa4::prefill_proj_block_q(), 1);
+    if (split && !set_split(p, prefill_workspace(args, true), workspace, workspace_bytes))
+      return IFA4_EWORKSPACE;
+  }
+  const hipError_t e = ifa4::launch_prefill(p, args->head_dim, args->qkv_dtype,
+                                            static_cast<hipStream_t>(stream));
+  return e == hipSuccess ? IFA4_OK : IFA4_ELAUNCH;
 }
 
 // Top-left causal decode (Lq = 1) sees key 0 only.
@@ -448,55 +515,27 @@ int32_t ifa4_prefill_fwd_ws(const ifa4_args* args, void* workspace, size_t works
   ifa4::PrefillParams p = make_prefill_params(args);
   const PrefillWorkspace w = prefill_workspace(args);
   set_tiles(p, args, ifa4::prefill_block_q(), w.pack);
-  if (w.total() > 0) {
-    if (workspace == nullptr || workspace_bytes < (size_t)w.total() || !aligned(workspace, 256))
-      return IFA4_EWORKSPACE;
-    p.chunk_tiles = w.split.chunk_tiles;
-    p.n_chunks = w.split.n_chunks;
-    p.seen_chunks = w.split.seen_chunks;
-    p.part_o = static_cast<float*>(workspace);
-    p.part_lse = reinterpret_cast<float*>(static_cast<char*>(workspace) + w.o_bytes);
-  }
+  if (!set_split(p, w, workspace, workspace_bytes)) return IFA4_EWORKSPACE;
   const hipError_t e = ifa4::launch_prefill(p, args->head_dim, args->qkv_dtype,
                                             static_cast<hipStream_t>(stream));
   return e == hipSuccess ? IFA4_OK : IFA4_ELAUNCH;
 }
 
 int32_t ifa4_prefill_rproj_fwd(const ifa4_args* args, const ifa4_rel_proj* pr, void* stream) {
-  if (args == nullptr || pr == nullptr || pr->struct_size != sizeof(ifa4_rel_proj))
-    return IFA4_EINVAL;
-  if (pr->d_rel != 16) return IFA4_EUNSUPPORTED;
-  if (args->rel_dtype != IFA4_BF16 && args->rel_dtype != IFA4_FP32) return IFA4_EUNSUPPORTED;
-  if (pr->r_stride_t < 0 || pr->r_stride_h < 0) return IFA4_EINVAL;
-  // The rel arguments of ifa4_args describe r here: checked below, not by check_args.
-  ifa4_args b = *args;
-  b.rel = pr->r;
-  b.rel_stride_t = 0;
-  b.rel_stride_h = 0;
-  const int32_t st = check_args(&b);
-  if (st != IFA4_OK) return st;
-  if (args->batch == 0 || args->max_seqlen_q == 0) return IFA4_OK;
-  if (args->rel_extent > 0) {
-    const int64_t esize = args->rel_dtype == IFA4_FP32 ? 4 : 2;
-    if (pr->r == nullptr || pr->wt == nullptr || !aligned(pr->r, esize) || !aligned(pr->wt, 16))
-      return IFA4_EINVAL;
-    if (pr->r_stride_t != 0 && pr->r_stride_t < 16) return IFA4_EUNSUPPORTED;
-    if (((int64_t)args->max_seqlen_q + ifa4::prefill_proj_block_q()) * pr->r_stride_t * esize >=
-            (int64_t(1) << 31) ||
-        (int64_t)args->rel_width * 64 >= (int64_t(1) << 31))
-      return IFA4_EUNSUPPORTED;
-  }
-  ifa4::PrefillParams p = make_prefill_params(&b);
-  p.rel = pr->r;
-  p.rel_st = pr->r_stride_t;
-  p.rel_sh = pr->r_stride_h;
-  p.wt = args->rel_extent > 0 ? pr->wt : nullptr;  // no bias at all: the plain kernel
-  if (p.wt != nullptr) {
-    set_tiles(p, args, ifa4::prefill_proj_block_q(), 1);
-  }
-  const hipError_t e = ifa4::launch_prefill(p, args->head_dim, args->qkv_dtype,
-                                            static_cast<hipStream_t>(stream));
-  return e == hipSuccess ? IFA4_OK : IFA4_ELAUNCH;
+  return run_rproj(args, pr, false, nullptr, 0, stream);
+}
+
+size_t ifa4_prefill_rproj_workspace_bytes(const ifa4_args* args, const ifa4_rel_proj* pr) {
+  ifa4_args b;
+  if (check_rproj(args, pr, &b) != IFA4_OK || args->batch == 0 || args->max_seqlen_q == 0 ||
+      args->rel_extent == 0)
+    return 0;
+  return (size_t)prefill_workspace(args, true).total();
+}
+
+int32_t ifa4_prefill_rproj_fwd_ws(const ifa4_args* args, const ifa4_rel_proj* pr, void* workspace,
+                                  size_t workspace_bytes, void* stream) {
+  return run_rproj(args, pr, true, workspace, workspace_bytes, stream);
 }
 
 int32_t ifa4_prefill_count_tiles(const ifa4_args* args, const int32_t* cu_q, const int32_t* cu_k,

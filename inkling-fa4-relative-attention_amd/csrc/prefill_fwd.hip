@@ -1449,6 +1449,7 @@ __global__ __launch_bounds__(kMergeThreads) void prefill_merge_kernel(PrefillPar
         l > 0.f ? (m + __log2f(l)) * kLn2 : -INFINITY;
 }
 
+static_assert(ProjShape::kBlockK == Shape::kBlockK, "one merge kernel for both");
 template <typename Sh, int D, typename Tag, int GROUPS>
 void launch_merge(const PrefillParams& p, hipStream_t stream) {
   constexpr int kRows = kMergeThreads / 32 / GROUPS;
@@ -1501,20 +1502,18 @@ hipError_t launch_prefill_t(const PrefillParams& p_in, hipStream_t stream) {
   if (blocks <= 0) return hipSuccess;
   hipLaunchKernelGGL((prefill_fwd_kernel<Sh, D, Tag, Rel, kProj, kTab, kPack>), dim3((unsigned)blocks),
                      dim3(Sh::kThreads), 0, stream, p);
-  if constexpr (!kProj) {  // the fused projection never splits
-    if (p.chunk_tiles > 0) {
-      const hipError_t e = hipGetLastError();
-      if (e != hipSuccess) return e;
-      // Groups pay where a call has few rows of many chunks: the rounds of a row
-      // are then all the merge waits for.  With many rows more workgroups cost
-      // more.  Whole calls, 1 / 2 / 8 groups (one box, us): 32 rows x up to 32
-      // chunks 19.3 / 17.2 / 15.5, 720 x 36 28.7 / 27.6 / 26.9, 1.8K x 36 32.5 / 31.5 /
-      // 31.2, 2K x 4 13.0 / 13.4 / 14.4, 9.3K x 6 63.8 / 65.8 / 71.5.
-      if (p.seen_chunks > 8 && (int64_t)p.n_heads * p.total_q <= 2048)
-        launch_merge<Sh, D, Tag, 8>(p, stream);
-      else
-        launch_merge<Sh, D, Tag, 1>(p, stream);
-    }
+  if (p.chunk_tiles > 0) {
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    // Groups pay where a call has few rows of many chunks: the rounds of a row
+    // are then all the merge waits for.  With many rows more workgroups cost
+    // more.  Whole calls, 1 / 2 / 8 groups (one box, us): 32 rows x up to 32
+    // chunks 19.3 / 17.2 / 15.5, 720 x 36 28.7 / 27.6 / 26.9, 1.8K x 36 32.5 / 31.5 /
+    // 31.2, 2K x 4 13.0 / 13.4 / 14.4, 9.3K x 6 63.8 / 65.8 / 71.5.
+    if (p.seen_chunks > 8 && (int64_t)p.n_heads * p.total_q <= 2048)
+      launch_merge<Shape, D, Tag, 8>(p, stream);
+    else
+      launch_merge<Shape, D, Tag, 1>(p, stream);
   }
   return hipGetLastError();
 }

@@ -269,6 +269,22 @@ inline int64_t prefill_chunk_count(int64_t lq, int64_t lk, const PrefillMasks& m
   return n;
 }
 
+// The slots a split may fill and when it pays, per kernel.
+struct SplitRule {
+  int64_t slots;       // resident workgroups
+  int64_t small_grid;  // grids up to here split whatever the range
+  int64_t min_saved;   // else a chunk of at most half of it, or this many tiles saved
+};
+constexpr SplitRule kPrefillSplitRule = {kPrefillSlots, kPrefillSplitSmallGrid,
+                                         kPrefillSplitMinSaved};
+// Fused projection: one 256-row workgroup per CU, and a tile in the bias band costs
+// it about 3 us, so any underfilled grid splits when that saves four tiles.  Whole
+// calls without and with the split (one box, us, Hq 8 / Hkv 2, d 128, extent 1024,
+// bf16 r): 2 x 900..2100 tokens 86.0 -> 60.6, 1 x 1000 66.5 -> 33.2, 1 x 3000 117 -> 90,
+// 3 x 100..600 over 300..2000 keys bottom-right 102.5 -> 61.8, 3 x 2000 98.7 -> 93.0
+// (98.0 when 16 tiles had to be saved), 6 x 1200 (240 workgroups, no split) 76.
+constexpr SplitRule kProjSplitRule = {256, 256, 4};
+
 // bottom_right: the queries are the last of their sequence's keys.  The estimate
 // takes the longest cache for every sequence and, without a window, every key for
 // every query (the causal mask takes max_q keys at most).  With a window the
@@ -280,7 +296,8 @@ inline int64_t prefill_chunk_count(int64_t lq, int64_t lk, const PrefillMasks& m
 inline PrefillSplit prefill_split_for(int64_t batch, int64_t n_heads, int64_t max_q,
                                       int64_t max_k, bool causal, int64_t window_left,
                                       bool bottom_right, bool no_prune, int32_t block_q,
-                                      int32_t block_k, int32_t forced_chunk) {
+                                      int32_t block_k, int32_t forced_chunk,
+                                      const SplitRule& rule = kPrefillSplitRule) {
   PrefillSplit s{0, 1, 1};
   if (batch <= 0 || max_q <= 0 || max_k <= 0) return s;
   const PrefillMasks masks{causal && !(bottom_right && window_left < 0), window_left,
@@ -290,11 +307,10 @@ inline PrefillSplit prefill_split_for(int64_t batch, int64_t n_heads, int64_t ma
   int64_t chunk = forced_chunk;
   if (chunk <= 0) {
     const int64_t grid = (max_q + block_q - 1) / block_q * n_heads * batch;
-    if (grid > kPrefillSplitMaxGrid) return s;
-    if (grid > kPrefillSplitSmallGrid && tmax < kPrefillSplitWideMinTiles) return s;
+    if (grid >= rule.slots || grid > kPrefillSplitMaxGrid) return s;
+    if (grid > rule.small_grid && tmax < kPrefillSplitWideMinTiles) return s;
     const int64_t balanced =
-        ((total * batch * n_heads + kPrefillSlots - 1) / kPrefillSlots * kPrefillChunkPct + 99) /
-        100;
+        ((total * batch * n_heads + rule.slots - 1) / rule.slots * kPrefillChunkPct + 99) / 100;
     chunk = balanced > kPrefillMinChunk ? balanced : kPrefillMinChunk;
     if (IFA4_PREFILL_CHUNK_FIT && chunk < tmax) {
       // Chunks of the balanced share can number a little more than the slots
@@ -303,7 +319,7 @@ inline PrefillSplit prefill_split_for(int64_t batch, int64_t n_heads, int64_t ma
       // (binary search; the count falls as the chunk grows).
       auto fits = [&](int64_t c) {
         return prefill_chunk_count(max_q, max_k, masks, block_q, block_k, c) * batch * n_heads <=
-               kPrefillSlots;
+               rule.slots;
       };
       if (!fits(chunk)) {
         // hi = tmax: one chunk per query tile whose range starts at key 0, which
@@ -319,7 +335,7 @@ inline PrefillSplit prefill_split_for(int64_t batch, int64_t n_heads, int64_t ma
     }
     // A split that shortens the longest range by little does not repay the
     // chunks' partials and the merge pass.
-    if (tmax <= chunk || (2 * chunk > tmax && tmax - chunk < kPrefillSplitMinSaved)) return s;
+    if (tmax <= chunk || (2 * chunk > tmax && tmax - chunk < rule.min_saved)) return s;
   }
   // chunk slots: enough for a query tile that meets every key tile (chunks are
   // aligned to multiples of `chunk` tiles on the key axis), so the grid and the

@@ -182,7 +182,13 @@ std::tuple<at::Tensor, at::Tensor> fwd_rproj(const at::Tensor& q, const at::Tens
     a.lse_stride_h = lse.stride(0);
   }
   const hipStream_t stream = c10::hip::getCurrentHIPStream(q.device().index()).stream();
-  check_status(ifa4_prefill_rproj_fwd(&a, &pr, stream), "fwd_rproj");
+  // split-KV workspace when the tile table splits this call (0 bytes otherwise)
+  const size_t ws_bytes = ifa4_prefill_rproj_workspace_bytes(&a, &pr);
+  at::Tensor ws = ws_bytes > 0 ? at::empty({(int64_t)ws_bytes}, q.options().dtype(at::kByte))
+                               : at::Tensor();
+  check_status(ifa4_prefill_rproj_fwd_ws(&a, &pr, ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes,
+                                         stream),
+               "fwd_rproj");
   return {out, lse};
 }
 

@@ -96,6 +96,10 @@ SIGNATURES = {
     "ifa4_prefill_fwd_ws": (_c_int32, [_P_ARGS, _vp, ctypes.c_size_t, _vp]),
     "ifa4_prefill_tile": (_c_int32, [_P_ARGS, _P_TILE]),
     "ifa4_prefill_rproj_fwd": (_c_int32, [_P_ARGS, ctypes.POINTER(Ifa4RelProj), _vp]),
+    "ifa4_prefill_rproj_workspace_bytes": (ctypes.c_size_t,
+                                           [_P_ARGS, ctypes.POINTER(Ifa4RelProj)]),
+    "ifa4_prefill_rproj_fwd_ws": (_c_int32, [_P_ARGS, ctypes.POINTER(Ifa4RelProj), _vp,
+                                             ctypes.c_size_t, _vp]),
     "ifa4_prefill_count_tiles": (_c_int32, [_P_ARGS, _P_I32, _P_I32, _P_I64, _P_I64]),
     "ifa4_decode_workspace_bytes": (ctypes.c_size_t, [_P_ARGS]),
     "ifa4_decode_tile": (_c_int32, [_P_ARGS, _P_TILE]),
