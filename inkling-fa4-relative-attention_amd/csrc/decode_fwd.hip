@@ -49,6 +49,11 @@
 // column keeps the one of its own kv head; PV adds each head's Vᵀ times P with
 // the other head's columns zeroed.
 //
+// Short caches (ifa4::decode_whole) take neither pass: the same stream code in a
+// workgroup of kNw waves per segment, one launch (kNw > 0).  What bounds such a
+// call is the chain of memory rounds (bounds, block table, K/V of each step) and
+// the launches; see the figures at decode_whole.
+//
 // Pass 2 (decode_combine_kernel): per (head, sequence) merge of the segment's
 // partials by log-sum-exp (16 part groups of a workgroup each merge online,
 // then meet in LDS); writes out (q dtype) and lse (natural log).
@@ -312,8 +317,13 @@ __device__ __forceinline__ int step_key0(const Cursor& cu) {
   return (cu.kbeg & ~(kStep - 1)) + cu.step * kStep;
 }
 
-template <int D, typename Tag, int G, bool kPaged, int Eb, bool kPair>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPair ? IFA4_DECODE_WPE_PAIR : IFA4_DECODE_WPE, 8))) void decode_stream_kernel(DecodeParams p) {
+// kNw = 0: the stream-K pass.  kNw > 0: short caches in one launch; a workgroup
+// of kNw waves takes one whole segment, wave w its steps w, w + kNw, ..., and the
+// waves' partials meet in LDS (no workspace, no combine pass).
+template <int D, typename Tag, int G, bool kPaged, int Eb, bool kPair, int kNw>
+__global__ __launch_bounds__(64 * (kNw > 0 ? kNw : 1)) __attribute__((amdgpu_waves_per_eu(
+    kPair ? IFA4_DECODE_WPE_PAIR : kNw > 0 && G > 8 ? 1 : IFA4_DECODE_WPE, 8))) void
+decode_stream_kernel(DecodeParams p) {
   using E = Elem<Tag>;
   using S = DecodeShape<D, Eb>;
   static_assert(!kPair || (Eb == 1 && D == 128 && G >= 2 && G <= 8), "pair mode: fp8, d 128");
@@ -322,24 +332,33 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPair ? IFA4
 
   // 16-bit tiles (K padded rows, V swizzled), or in pair mode the fp8 tiles
   // (K: 16 rows, V: kStep rows, kPairPitch bytes each)
-  __shared__ __align__(16) uint16_t k_lds[kPair ? 16 * kPairPitch / 2 : kStep * S::kPitch];
-  __shared__ __align__(16) uint16_t v_lds[kPair ? kStep * kPairPitch / 2 : kStep * D];
+  constexpr int kW = kNw > 0 ? kNw : 1;  // waves of the workgroup, each with its own tiles
+  __shared__ __align__(16)
+      uint16_t k_tiles[kW][kPair ? 16 * kPairPitch / 2 : kStep * S::kPitch];
+  __shared__ __align__(16) uint16_t v_tiles[kW][kPair ? kStep * kPairPitch / 2 : kStep * D];
+  const int wv = kNw > 0 ? (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  auto& k_lds = k_tiles[wv];
+  auto& v_lds = v_tiles[wv];
   using Q = DecodeQ<D, G>;
   constexpr int kNbuf = kPair ? IFA4_DECODE_NBUF_PAIR : Eb == 1 ? IFA4_DECODE_NBUF_FP8 : 2;
-  // Loads of the next step in flight while a step computes (pair mode).  The
-  // other formats issue them only while the wave's range lasts; the compiler
+  // Loads of the next step in flight while a step computes (pair mode, and the
+  // one-launch form, whose few waves have nothing else in flight).  The other
+  // formats issue them only while the wave's range lasts; the compiler
   // then merges the two paths' counts and its wait before a step's LDS writes
   // also covers the next step's loads, so each wave computes with no loads in
   // flight -- measured faster for them at their wave counts.
-  constexpr bool kOverlap = kPair && IFA4_DECODE_PAIR_OVERLAP;
+  constexpr bool kOverlap = (kPair && IFA4_DECODE_PAIR_OVERLAP) || kNw > 0;
   static_assert(kNbuf >= 2 && kNbuf <= 3, "two or three step buffers");
   // One Q slot per step buffer: the segments of the steps in flight hold
   // distinct slots, so a slot is rewritten only after its segment's Q was read.
-  __shared__ __align__(1024) uint16_t q_lds[kNbuf][Q::kElems];
+  // (one launch: a single segment, one slot)
+  constexpr int kSlots = kNw > 0 ? 1 : kNbuf;
+  __shared__ __align__(1024) uint16_t q_slots[kW][kSlots][Q::kElems];
+  auto& q_lds = q_slots[wv];
 
   const int w = blockIdx.x;
-  const int W = p.n_waves;
-  const int lane = threadIdx.x;
+  [[maybe_unused]] const int W = p.n_waves;
+  const int lane = kNw > 0 ? threadIdx.x & 63 : threadIdx.x;
   const int r = lane / L::kLpr;  // row layout
   const int c = lane % L::kLpr;
   const int n = lane & 15;       // S^T layout
@@ -349,16 +368,20 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPair ? IFA4
 
   // ---- total units T (every wave derives the same), this wave's range ----------
   // A wave computes the steps that start inside its range of units.
-  SeqChunk ch = load_chunk<kPaged>(p, 0, 0, lane);
-  int total = ch.total_incl;
-  for (int b = 64; b < p.batch; b += 64) total = load_chunk<kPaged>(p, b, total, lane).total_incl;
-  const int T = hkv * total;
-  if (T == 0) return;
-  const int P = (T + W - 1) / W;
-  const int g0 = w * P;
-  const int g1 = min(g0 + P, T);
-  if (g0 >= g1) return;
-  if (p.batch > 64) ch = load_chunk<kPaged>(p, 0, 0, lane);
+  SeqChunk ch{};
+  [[maybe_unused]] int P = 1, g0 = 0, g1 = 0;
+  if constexpr (kNw == 0) {
+    ch = load_chunk<kPaged>(p, 0, 0, lane);
+    int total = ch.total_incl;
+    for (int b = 64; b < p.batch; b += 64) total = load_chunk<kPaged>(p, b, total, lane).total_incl;
+    const int T = hkv * total;
+    if (T == 0) return;
+    P = (T + W - 1) / W;
+    g0 = w * P;
+    g1 = min(g0 + P, T);
+    if (g0 >= g1) return;
+    if (p.batch > 64) ch = load_chunk<kPaged>(p, 0, 0, lane);
+  }
 
   // Cursor of the first step that starts at global unit gu or later (gu only
   // moves forward; the chunk follows it).  Returns steps == 0 if there is none
@@ -598,7 +621,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPair ? IFA4
       l_run = 0.f;
 #pragma unroll
       for (int db = 0; db < S::kDBlocks; ++db) o[db] = f32x4_t{};
-      if (cu.step == 0 && lane == 0) {
+      if (kNw == 0 && cu.step == 0 && lane == 0) {
         // this wave holds the segment's first step: record the covering waves
         p.ws_meta[2 * cu.seg] = w;
         p.ws_meta[2 * cu.seg + 1] = (cu.seg_u0 + step_unit(cu, cu.steps - 1)) / P;
@@ -826,7 +849,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPair ? IFA4
     }
     wave_lds_sync();  // k_lds / v_lds are rewritten by the next step
 
-    if (!last) return;
+    if (kNw > 0 || !last) return;
     // ---- partial of (segment, wave): normalise, store ------------------------------
     const float l_tot = add_xor32(add_xor16(l_run));  // per head n, all g
     const float inv = l_tot > 0.f ? p.v_scale / l_tot : 0.f;  // V scale (1 for 16-bit V)
@@ -841,26 +864,83 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPair ? IFA4
   Cursor cur[kNbuf];
   bool live[kNbuf];
   u32x4_t kbuf[kNbuf][L::kLoads], vbuf[kNbuf][L::kLoads];
-  cur[0] = locate(g0);
-  if (cur[0].steps == 0) return;
-  if (cur[0].seg_u0 + step_unit(cur[0], cur[0].step) >= g1) {
-    // No step starts in this wave's range.  If the range lies inside the
-    // segment (between two of its steps' starts), the segment's partials run
-    // over this wave's slot too: an empty one (nothing seen) goes there.
-    if (g0 >= cur[0].seg_u0) {
-#pragma unroll
-      for (int db = 0; db < S::kDBlocks; ++db) o[db] = f32x4_t{};
-      put_partial(cur[0].seg + w, 0.f, -INFINITY);
+  if constexpr (kNw > 0) {
+    // ---- one whole segment: this workgroup's (sequence, kv head) ------------------
+    const int seq = w / hkv;
+    const SeqBounds bq = seq_bounds(p.cu_q, seq, p.total_q);
+    Cursor cu;
+    cu.seq = seq;
+    cu.kvh = w - seq * hkv;
+    cu.seg = w;
+    cu.qs = bq.start;
+    cu.ks = 0;
+    if constexpr (kPaged) {
+      cu.lk = paged_len(p, seq);
+    } else {
+      const SeqBounds bk = seq_bounds(p.cu_k, seq, p.total_k);
+      cu.ks = bk.start;
+      cu.lk = bk.len;
     }
-    return;
+    if (bq.len != 1) {
+      // not one query token: its query rows, if any, get out = 0, lse = -inf
+      constexpr int kRowThreads = D / 8;
+      const int d = 8 * ((int)threadIdx.x % kRowThreads);
+      for (int row = (int)threadIdx.x / kRowThreads; row < bq.len * g_act;
+           row += 64 * kW / kRowThreads) {
+        const int64_t t = bq.start + row / g_act;
+        const int head = cu.kvh * g_act + row % g_act;
+        *reinterpret_cast<u32x4_t*>(static_cast<uint16_t*>(p.out) + t * p.o_st +
+                                    (int64_t)head * p.o_sh + d) = u32x4_t{0u, 0u, 0u, 0u};
+        if (p.lse != nullptr && d == 0) p.lse[(int64_t)head * p.lse_sh + t] = -INFINITY;
+      }
+      return;
+    }
+    const KeyRange kr = decode_keys(p, cu.lk);
+    cu.kbeg = kr.kbeg;
+    cu.kend = kr.kend;
+    cu.steps = seq_steps(1, kr);
+    cu.nb = cu.steps;
+    cu.units = 0;
+    cu.seg_u0 = 0;
+    cu.slot = 0;
+    cu.step = wv;
+    cur[0] = cu;
+#pragma unroll
+    for (int db = 0; db < S::kDBlocks; ++db) o[db] = f32x4_t{};
+    live[0] = wv < cu.steps;
+  } else {
+    cur[0] = locate(g0);
+    if (cur[0].steps == 0) return;
+    if (cur[0].seg_u0 + step_unit(cur[0], cur[0].step) >= g1) {
+      // No step starts in this wave's range.  If the range lies inside the
+      // segment (between two of its steps' starts), the segment's partials run
+      // over this wave's slot too: an empty one (nothing seen) goes there.
+      if (g0 >= cur[0].seg_u0) {
+  #pragma unroll
+        for (int db = 0; db < S::kDBlocks; ++db) o[db] = f32x4_t{};
+        put_partial(cur[0].seg + w, 0.f, -INFINITY);
+      }
+      return;
+    }
   }
   cur[0].first = true;
-  load_q(cur[0]);
-  load(kbuf[0], vbuf[0], cur[0], true);
-  live[0] = true;
+  if constexpr (kNw > 0) {
+    if (live[0]) load_q(cur[0]);
+    load(kbuf[0], vbuf[0], cur[0], live[0]);
+  } else {
+    load_q(cur[0]);
+    load(kbuf[0], vbuf[0], cur[0], true);
+    live[0] = true;
+  }
   // Next cursor after `cu`, with its Q slot (a new segment takes the next slot,
   // whose earlier segment's Q was read into registers kNbuf - 1 steps before).
   auto next = [&](const Cursor& cu) -> Cursor {
+    if constexpr (kNw > 0) {
+      Cursor nx = cu;
+      nx.step = cu.step + kNw;
+      nx.first = false;
+      return nx;
+    }
     if (cu.step + 1 < cu.steps) {
       Cursor nx = cu;
       nx.step = cu.step + 1;
@@ -877,7 +957,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPair ? IFA4
     live[j] = live[jp];
     if (live[j]) {
       cur[j] = next(cur[jp]);
-      live[j] = cur[j].steps > 0 && cur[j].seg_u0 + step_unit(cur[j], cur[j].step) < g1;
+      if constexpr (kNw > 0)
+        live[j] = cur[j].step < cur[j].steps;
+      else
+        live[j] = cur[j].steps > 0 && cur[j].seg_u0 + step_unit(cur[j], cur[j].step) < g1;
     }
     if constexpr (kOverlap) {
       // every path issues the step's loads (past the range through empty
@@ -891,7 +974,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPair ? IFA4
   };
 #pragma unroll
   for (int j = 1; j < kNbuf - 1; ++j) issue(j, j - 1);
-  bool more = true;
+  bool more = kNw > 0 ? live[0] : true;
   while (more) {
 #pragma unroll
     for (int j = 0; j < kNbuf; ++j) {
@@ -911,9 +994,59 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPair ? IFA4
       }
     }
   }
+  if constexpr (kNw > 0) {
+    // ---- merge the waves' partials ------------------------------------------------
+    // Each wave leaves its unnormalised O in its own K tile (no other wave reads or
+    // writes that before the barrier), [head][D] fp32; a thread then owns a 16-byte
+    // chunk of a head's row over all waves.
+    constexpr int kHeads = G < 16 ? G : 16;
+    static_assert(kHeads * D * 4 <= (int)sizeof(k_tiles[0]) + (int)sizeof(v_tiles[0]),
+                  "a wave's partial fits its tiles");
+    constexpr bool kInK = kHeads * D * 4 <= (int)sizeof(k_tiles[0]);
+    __shared__ float part_m[kW][kHeads], part_l[kW][kHeads];
+    const float l_tot = add_xor32(add_xor16(l_run));
+    float* const mine = reinterpret_cast<float*>(kInK ? k_lds : v_lds);
+    if (n < g_act) {
+#pragma unroll
+      for (int db = 0; db < S::kDBlocks; ++db)
+        *reinterpret_cast<f32x4_t*>(mine + n * D + 16 * db + 4 * g) = o[db];
+      if (g == 0) {
+        part_m[wv][n] = m_run;
+        part_l[wv][n] = l_tot;
+      }
+    }
+    __syncthreads();
+    constexpr int kRowChunks = D / 4;
+    for (int c4 = threadIdx.x; c4 < g_act * kRowChunks; c4 += 64 * kW) {
+      const int h = c4 / kRowChunks, d = 4 * (c4 % kRowChunks);
+      float mt = part_m[0][h];
+#pragma unroll
+      for (int i = 1; i < kW; ++i) mt = fmaxf(mt, part_m[i][h]);
+      const float mu = mt == -INFINITY ? 0.f : mt;
+      float lt = 0.f;
+      f32x4_t out{};
+#pragma unroll
+      for (int i = 0; i < kW; ++i) {
+        const float a = fast_exp2(part_m[i][h] - mu);
+        lt += a * part_l[i][h];
+        out += a * *reinterpret_cast<const f32x4_t*>(
+                       reinterpret_cast<const float*>(kInK ? k_tiles[i] : v_tiles[i]) + h * D + d);
+      }
+      const float inv = lt > 0.f ? p.v_scale / lt : 0.f;
+      const int head = cur[0].kvh * g_act + h;
+      uint16_t* dst = static_cast<uint16_t*>(p.out) + (int64_t)cur[0].qs * p.o_st +
+                      (int64_t)head * p.o_sh + d;
+      *reinterpret_cast<u32x2_t*>(dst) =
+          u32x2_t{E::pack2(out[0] * inv, out[1] * inv), E::pack2(out[2] * inv, out[3] * inv)};
+      if (p.lse != nullptr && d == 0)
+        p.lse[(int64_t)head * p.lse_sh + cur[0].qs] =
+            lt > 0.f ? (mt + __log2f(lt)) * kLn2 : -INFINITY;
+    }
+  }
 }
 
 constexpr int kCombineWaves = 8;
+constexpr int kWholeWaves = 8;  // waves of a one-launch workgroup
 
 // SPLIT workgroups per (head, sequence), workgroup z over the 16-byte chunks
 // [z, z + 1) * D / (4 SPLIT) of the row.  Two dependent memory rounds: the
@@ -1015,40 +1148,48 @@ __global__ __launch_bounds__(64 * kCombineWaves) void decode_combine_kernel(Deco
   }
 }
 
-template <int D, typename Tag, int G>
-hipError_t launch_decode_g(const DecodeParams& p, hipStream_t stream) {
-  if (p.n_waves > 0) {
-    const dim3 grid(p.n_waves), block(64);
-    if (p.kv_pair) {
-      // the host pairs kv heads only for fp8 caches of d 128 whose pairs hold
-      // 2..8 query heads
-      if constexpr (D == 128 && G >= 2 && G <= 8) {
-        if (!p.kv_fp8) return hipErrorInvalidValue;
-        if (p.block_table != nullptr)
-          hipLaunchKernelGGL((decode_stream_kernel<D, Tag, G, true, 1, true>), grid, block, 0,
-                             stream, p);
-        else
-          hipLaunchKernelGGL((decode_stream_kernel<D, Tag, G, false, 1, true>), grid, block, 0,
-                             stream, p);
-      } else {
-        return hipErrorInvalidValue;
-      }
-    } else if (p.kv_fp8) {
+template <int D, typename Tag, int G, int kNw>
+hipError_t launch_decode_pass(const DecodeParams& p, hipStream_t stream) {
+  const dim3 grid(kNw > 0 ? p.batch * p.kv_heads : p.n_waves), block(64 * (kNw > 0 ? kNw : 1));
+  if (p.kv_pair) {
+    // the host pairs kv heads only for fp8 caches of d 128 whose pairs hold
+    // 2..8 query heads
+    if constexpr (D == 128 && G >= 2 && G <= 8) {
+      if (!p.kv_fp8) return hipErrorInvalidValue;
       if (p.block_table != nullptr)
-        hipLaunchKernelGGL((decode_stream_kernel<D, Tag, G, true, 1, false>), grid, block, 0,
+        hipLaunchKernelGGL((decode_stream_kernel<D, Tag, G, true, 1, true, kNw>), grid, block, 0,
                            stream, p);
       else
-        hipLaunchKernelGGL((decode_stream_kernel<D, Tag, G, false, 1, false>), grid, block, 0,
+        hipLaunchKernelGGL((decode_stream_kernel<D, Tag, G, false, 1, true, kNw>), grid, block, 0,
                            stream, p);
     } else {
-      if (p.block_table != nullptr)
-        hipLaunchKernelGGL((decode_stream_kernel<D, Tag, G, true, 2, false>), grid, block, 0,
-                           stream, p);
-      else
-        hipLaunchKernelGGL((decode_stream_kernel<D, Tag, G, false, 2, false>), grid, block, 0,
-                           stream, p);
+      return hipErrorInvalidValue;
     }
-    hipError_t e = hipGetLastError();
+  } else if (p.kv_fp8) {
+    if (p.block_table != nullptr)
+      hipLaunchKernelGGL((decode_stream_kernel<D, Tag, G, true, 1, false, kNw>), grid, block, 0,
+                         stream, p);
+    else
+      hipLaunchKernelGGL((decode_stream_kernel<D, Tag, G, false, 1, false, kNw>), grid, block, 0,
+                         stream, p);
+  } else {
+    if (p.block_table != nullptr)
+      hipLaunchKernelGGL((decode_stream_kernel<D, Tag, G, true, 2, false, kNw>), grid, block, 0,
+                         stream, p);
+    else
+      hipLaunchKernelGGL((decode_stream_kernel<D, Tag, G, false, 2, false, kNw>), grid, block, 0,
+                         stream, p);
+  }
+  return hipGetLastError();
+}
+
+template <int D, typename Tag, int G>
+hipError_t launch_decode_g(const DecodeParams& p, hipStream_t stream) {
+  // groups above 8: half the waves, whose Q rows and tiles fill the LDS
+  if (p.whole)
+    return launch_decode_pass<D, Tag, G, G < 16 ? kWholeWaves : kWholeWaves / 2>(p, stream);
+  if (p.n_waves > 0) {
+    const hipError_t e = launch_decode_pass<D, Tag, G, 0>(p, stream);
     if (e != hipSuccess) return e;
   }
   // Splits of the combine: enough part groups that the parts of a segment

@@ -424,6 +424,13 @@ int32_t run_decode(const ifa4_args* args, const ifa4_paged_kv* kv, const ifa4_kv
   p.window_left = args->window_left < (1 << 30) ? args->window_left : (1 << 30);
   p.rel_dtype = args->rel_dtype;
   p.n_waves = decode_waves(args, qt != nullptr, kv != nullptr);
+  // steps of the longest cache: its visible keys, and one more for the partial
+  // step a window may begin with
+  int64_t keys = key0_only(args) ? (args->max_seqlen_k > 0 ? 1 : 0) : args->max_seqlen_k;
+  if (p.bottom_right && p.window_left >= 0 && keys > p.window_left + ifa4::kDecodeStep)
+    keys = p.window_left + ifa4::kDecodeStep;
+  p.whole = ifa4::decode_whole((int64_t)args->batch * view.kv_heads, view.group,
+                               (keys + ifa4::kDecodeStep - 1) / ifa4::kDecodeStep);
   p.kv_fp8 = qt != nullptr ? 1 : 0;
   p.scale_log2 = args->softmax_scale * (qt != nullptr ? qt->k_scale : 1.f) * kLog2eHost;
   p.v_scale = qt != nullptr ? qt->v_scale : 1.f;

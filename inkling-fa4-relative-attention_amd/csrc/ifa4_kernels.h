@@ -86,6 +86,7 @@ struct DecodeParams {
   int32_t window_left;   // -1: none (only matters with bottom_right: top-left decode never masks)
   int32_t rel_dtype;
   int32_t n_waves;   // persistent waves of pass 1 (0: nothing to stream)
+  int32_t whole;     // 1: one launch, a workgroup per (sequence, kv head); no workspace
   int32_t kv_fp8;    // 1: K and V are fp8 (OCP e4m3), K scale folded into scale_log2
   // 1: each kv head of these params is a pair of adjacent fp8 kv heads (k_sh,
   // v_sh = 2 * head_dim, group = both heads' query heads), streamed as whole rows

@@ -119,6 +119,25 @@ inline bool decode_pairs(bool fp8, int64_t head_dim, int64_t kv_heads, int64_t g
          2 * group <= 8 && k_stride_h == head_dim && v_stride_h == head_dim;
 }
 
+// Short caches: one launch with a workgroup of 8 waves per (sequence, kv head)
+// (4 for groups above 8) instead of the stream and combine passes.  A wave's
+// steps wait for one another's loads (about 2 us each), so it pays up to three
+// steps a wave (a window of 512 keys is 17 steps), and up to four where the
+// segments alone fill the chip.  Two passes -> one launch (one box, us, Hq 8 /
+// Hkv 2, d 128; sequences x keys):
+//   bf16 1 x 512 14.1 -> 10.8, 64 x 512 18.2 -> 12.3, 128 x 256 20.0 -> 11.0, 128 x
+//   512 26.5 -> 15.3, 64 x 1024 24.7 -> 18.9, 128 x 1024 39.6 -> 25.4, but 16 x 1024
+//   14.1 -> 16.2, 16 x 2048 16.2 -> 27.0;
+//   paged 64 x 512 19.0 -> 13.5, paged fp8 64 x 512 18.2 -> 14.1, window 511 over
+//   200..6000 paged keys 24 sequences 15.9 -> 14.0, 64 20.8 -> 15.0; window 1023
+//   (33 steps) 16.9 -> 21.1.
+// With 4 waves a segment everything but 64 x 256 is slower (64 x 512 13.4, windows 18.5).
+inline bool decode_whole(int64_t segments, int64_t group, int64_t max_steps) {
+  const int64_t waves = group > 8 ? 4 : 8;
+  if (2 * max_steps <= 5 * waves) return true;
+  return max_steps <= 4 * waves && segments >= 128;
+}
+
 // kv_heads: as the kernel sees them (pairs when pair is set).
 inline int32_t decode_waves_for(int64_t batch, int64_t kv_heads, int64_t max_seqlen_k,
                                 bool key0_only, bool fp8, bool paged, bool pair = false) {
