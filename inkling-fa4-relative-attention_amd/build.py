@@ -84,7 +84,7 @@ def build_torch_binding():
            f"-I{INCLUDE}", f"-I{ROCM}/include"]
     cmd += [f"-I{p}" for p in inc]
     cmd += [f"-L{p}" for p in libdirs] + [f"-L{PKG}", f"-L{ROCM}/lib"]
-    cmd += ["-lifa4", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-lamdhip64",
+    cmd += ["-lifa4", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-lamdhip64",
             "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{ROCM}/lib"]
     _run(cmd)
     os.replace(tmp, out)

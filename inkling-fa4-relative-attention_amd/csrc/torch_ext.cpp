@@ -10,6 +10,7 @@
 // (src/inkling_fa4/triton_kernel.py:84-107); the Python layer (inkling_fa4.ops)
 // keeps the positional API and adds softmax_scale / return_lse.
 #include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <torch/library.h>
 #include <c10/hip/HIPStream.h>
 
@@ -26,6 +27,13 @@ int32_t dtype_code(at::ScalarType t) {
     case at::kFloat: return IFA4_FP32;
     default: return -1;
   }
+}
+
+// Uninitialised tensors on q's GPU from the caching allocator, without a dispatcher
+// round per tensor (the output, the LSE and the workspace of a call: 9.4 -> 8.4 us
+// of host time for a short prompt).
+at::Tensor empty_on(const at::Tensor& q, at::IntArrayRef sizes, at::ScalarType dtype) {
+  return at::Tensor(at::detail::empty_cuda(sizes, dtype, q.device(), std::nullopt));
 }
 
 void check_status(int32_t st, const char* what) {
@@ -121,9 +129,9 @@ std::tuple<at::Tensor, at::Tensor> fwd(const at::Tensor& q, const at::Tensor& k,
               "inkling_fa4.fwd: fp8 K/V is supported by decode only");
   ifa4_args a = make_args(q, k, v, rel, cu_q, cu_k, max_q, max_k, rel_extent, causal,
                           window_left, softmax_scale, flags);
-  at::Tensor out = at::empty_like(q, q.options().memory_format(at::MemoryFormat::Contiguous));
-  at::Tensor lse = return_lse ? at::empty({q.size(1), q.size(0)}, q.options().dtype(at::kFloat))
-                              : at::empty({0}, q.options().dtype(at::kFloat));
+  at::Tensor out = empty_on(q, q.sizes(), q.scalar_type());
+  at::Tensor lse = return_lse ? empty_on(q, {q.size(1), q.size(0)}, at::kFloat)
+                              : empty_on(q, {0}, at::kFloat);
   a.out = out.data_ptr();
   a.out_stride_t = out.stride(0);
   a.out_stride_h = out.stride(1);
@@ -135,7 +143,7 @@ std::tuple<at::Tensor, at::Tensor> fwd(const at::Tensor& q, const at::Tensor& k,
   const hipStream_t stream = c10::hip::getCurrentHIPStream(q.device().index()).stream();
   // split-KV workspace when the tile table splits this call (0 bytes otherwise)
   const size_t ws_bytes = ifa4_prefill_workspace_bytes(&a);
-  at::Tensor ws = ws_bytes > 0 ? at::empty({(int64_t)ws_bytes}, q.options().dtype(at::kByte))
+  at::Tensor ws = ws_bytes > 0 ? empty_on(q, {(int64_t)ws_bytes}, at::kByte)
                                : at::Tensor();
   check_status(ifa4_prefill_fwd_ws(&a, ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes, stream),
                "fwd");
@@ -171,9 +179,9 @@ std::tuple<at::Tensor, at::Tensor> fwd_rproj(const at::Tensor& q, const at::Tens
   pr.r_stride_t = r.stride(0);
   pr.r_stride_h = r.stride(1);
   pr.wt = wt.data_ptr<float>();
-  at::Tensor out = at::empty_like(q, q.options().memory_format(at::MemoryFormat::Contiguous));
-  at::Tensor lse = return_lse ? at::empty({q.size(1), q.size(0)}, q.options().dtype(at::kFloat))
-                              : at::empty({0}, q.options().dtype(at::kFloat));
+  at::Tensor out = empty_on(q, q.sizes(), q.scalar_type());
+  at::Tensor lse = return_lse ? empty_on(q, {q.size(1), q.size(0)}, at::kFloat)
+                              : empty_on(q, {0}, at::kFloat);
   a.out = out.data_ptr();
   a.out_stride_t = out.stride(0);
   a.out_stride_h = out.stride(1);
@@ -184,7 +192,7 @@ std::tuple<at::Tensor, at::Tensor> fwd_rproj(const at::Tensor& q, const at::Tens
   const hipStream_t stream = c10::hip::getCurrentHIPStream(q.device().index()).stream();
   // split-KV workspace when the tile table splits this call (0 bytes otherwise)
   const size_t ws_bytes = ifa4_prefill_rproj_workspace_bytes(&a, &pr);
-  at::Tensor ws = ws_bytes > 0 ? at::empty({(int64_t)ws_bytes}, q.options().dtype(at::kByte))
+  at::Tensor ws = ws_bytes > 0 ? empty_on(q, {(int64_t)ws_bytes}, at::kByte)
                                : at::Tensor();
   check_status(ifa4_prefill_rproj_fwd_ws(&a, &pr, ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes,
                                          stream),
@@ -201,9 +209,9 @@ std::tuple<at::Tensor, at::Tensor> decode(const at::Tensor& q, const at::Tensor&
                                           int64_t flags, double k_scale, double v_scale) {
   ifa4_args a = make_args(q, k, v, rel, cu_q, cu_k, max_q, max_k, rel_extent, causal,
                           window_left, softmax_scale, flags);
-  at::Tensor out = at::empty_like(q, q.options().memory_format(at::MemoryFormat::Contiguous));
-  at::Tensor lse = return_lse ? at::empty({q.size(1), q.size(0)}, q.options().dtype(at::kFloat))
-                              : at::empty({0}, q.options().dtype(at::kFloat));
+  at::Tensor out = empty_on(q, q.sizes(), q.scalar_type());
+  at::Tensor lse = return_lse ? empty_on(q, {q.size(1), q.size(0)}, at::kFloat)
+                              : empty_on(q, {0}, at::kFloat);
   a.out = out.data_ptr();
   a.out_stride_t = out.stride(0);
   a.out_stride_h = out.stride(1);
@@ -220,7 +228,7 @@ std::tuple<at::Tensor, at::Tensor> decode(const at::Tensor& q, const at::Tensor&
     check_status(kv_fp8 ? ifa4_decode_quant_fwd(&a, nullptr, &qt, nullptr, 0, nullptr)
                         : ifa4_decode_fwd(&a, nullptr, 0, nullptr),
                  "decode");
-  at::Tensor ws = at::empty({static_cast<int64_t>(ws_bytes) + 256}, q.options().dtype(at::kByte));
+  at::Tensor ws = empty_on(q, {static_cast<int64_t>(ws_bytes) + 256}, at::kByte);
   const uintptr_t base = reinterpret_cast<uintptr_t>(ws.data_ptr());
   void* aligned_ws = reinterpret_cast<void*>((base + 255) / 256 * 256);
   const hipStream_t stream = c10::hip::getCurrentHIPStream(q.device().index()).stream();
@@ -276,9 +284,9 @@ std::tuple<at::Tensor, at::Tensor> decode_paged(
   kv.num_blocks = static_cast<int32_t>(k_cache.size(0));
   kv.max_blocks_per_seq = static_cast<int32_t>(block_table.size(1));
 
-  at::Tensor out = at::empty_like(q, q.options().memory_format(at::MemoryFormat::Contiguous));
-  at::Tensor lse = return_lse ? at::empty({q.size(1), q.size(0)}, q.options().dtype(at::kFloat))
-                              : at::empty({0}, q.options().dtype(at::kFloat));
+  at::Tensor out = empty_on(q, q.sizes(), q.scalar_type());
+  at::Tensor lse = return_lse ? empty_on(q, {q.size(1), q.size(0)}, at::kFloat)
+                              : empty_on(q, {0}, at::kFloat);
   a.out = out.data_ptr();
   a.out_stride_t = out.stride(0);
   a.out_stride_h = out.stride(1);
@@ -294,7 +302,7 @@ std::tuple<at::Tensor, at::Tensor> decode_paged(
     check_status(kv_fp8 ? ifa4_decode_quant_fwd(&a, &kv, &qt, nullptr, 0, nullptr)
                         : ifa4_decode_paged_fwd(&a, &kv, nullptr, 0, nullptr),
                  "decode_paged");
-  at::Tensor ws = at::empty({static_cast<int64_t>(ws_bytes) + 256}, q.options().dtype(at::kByte));
+  at::Tensor ws = empty_on(q, {static_cast<int64_t>(ws_bytes) + 256}, at::kByte);
   const uintptr_t base = reinterpret_cast<uintptr_t>(ws.data_ptr());
   void* aligned_ws = reinterpret_cast<void*>((base + 255) / 256 * 256);
   const hipStream_t stream = c10::hip::getCurrentHIPStream(q.device().index()).stream();

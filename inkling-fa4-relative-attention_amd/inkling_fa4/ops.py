@@ -47,11 +47,12 @@ from . import _abi
 from ._native import ops as _ops
 
 
-def _resolve(q, k, n_heads, kv_heads, head_dim, softmax_scale):
-    if q.dim() != 3 or k.dim() != 3:
+def _resolve(q, k_shape, n_heads, kv_heads, head_dim, softmax_scale):
+    q_shape = q.shape
+    if len(q_shape) != 3 or len(k_shape) != 3:
         raise ValueError("q and k must be [tokens, heads, head_dim]")
-    hq, d = q.shape[1], q.shape[2]
-    hkv = k.shape[1]
+    hq, d = q_shape[1], q_shape[2]
+    hkv = k_shape[1]
     if n_heads is not None and n_heads != hq:
         raise ValueError(f"n_heads={n_heads} disagrees with q.shape[1]={hq}")
     if kv_heads is not None and kv_heads != hkv:
@@ -62,6 +63,28 @@ def _resolve(q, k, n_heads, kv_heads, head_dim, softmax_scale):
         raise ValueError(f"n_heads={hq} is not a multiple of kv_heads={hkv}")
     scale = (1.0 / d) if softmax_scale is None else float(softmax_scale)
     return scale
+
+
+_is_grad_enabled = torch.is_grad_enabled
+_overloads = {}
+
+
+def _call(name, *args):
+    """torch.ops.inkling_fa4.<name> with gradients off: the operators have no
+    backward, and their outputs never require one.  Small calls are bound by the
+    host (a short prompt or cache computes in less time than it takes to issue),
+    so the mode is switched, which costs a tenth of such a call, only when one of
+    the floating-point inputs (the first five arguments hold them) asks for a gradient."""
+    op = _overloads.get(name)
+    if op is None:
+        op = _overloads[name] = getattr(_ops(), name).default
+    if _is_grad_enabled():
+        q, k, v, rel, w = args[:5]
+        if (q.requires_grad or k.requires_grad or v.requires_grad or rel.requires_grad
+                or w.requires_grad):
+            with torch.no_grad():
+                return op(*args)
+    return op(*args)
 
 
 _FLAG_BOTTOM_RIGHT = 0x2  # IFA4_FLAG_BOTTOM_RIGHT
@@ -78,7 +101,6 @@ def _window_left(window_size):
     return left if left >= 0 else -1
 
 
-@torch.no_grad()
 def inkling_fa4_rel_attention(q, k, v, rel_logits, cu_seqlens_q, cu_seqlens_k,
                               max_seqlen_q, max_seqlen_k, rel_extent, causal=True,
                               window_size=(-1, -1), n_heads=None, kv_heads=None,
@@ -94,15 +116,14 @@ def inkling_fa4_rel_attention(q, k, v, rel_logits, cu_seqlens_q, cu_seqlens_k,
     i + Lk - Lq for the bias distance, causal mask and window); the default is
     the reference's top-left alignment.
     """
-    scale = _resolve(q, k, n_heads, kv_heads, head_dim, softmax_scale)
-    out, lse = _ops().fwd(q, k, v, rel_logits, cu_seqlens_q, cu_seqlens_k, int(max_seqlen_q),
-                          int(max_seqlen_k), int(rel_extent), bool(causal),
-                          _window_left(window_size), scale, bool(return_lse),
-                          _flag_bits(bottom_right, _flags))
+    scale = _resolve(q, k.shape, n_heads, kv_heads, head_dim, softmax_scale)
+    out, lse = _call("fwd", q, k, v, rel_logits, cu_seqlens_q, cu_seqlens_k, int(max_seqlen_q),
+                     int(max_seqlen_k), int(rel_extent), bool(causal),
+                     _window_left(window_size), scale, bool(return_lse),
+                     _flag_bits(bottom_right, _flags))
     return (out, lse) if return_lse else out
 
 
-@torch.no_grad()
 def inkling_fa4_rel_attention_decode(q, k, v, rel_logits, cu_seqlens_q, cu_seqlens_k,
                                      max_seqlen_q, max_seqlen_k, rel_extent, causal=True,
                                      window_size=(-1, -1), n_heads=None, kv_heads=None,
@@ -117,24 +138,22 @@ def inkling_fa4_rel_attention_decode(q, k, v, rel_logits, cu_seqlens_q, cu_seqle
     k / v may be torch.float8_e4m3fn (an FP8 KV cache, GQA groups up to 16):
     the keys and values are k * k_scale and v * v_scale.
     """
-    scale = _resolve(q, k, n_heads, kv_heads, head_dim, softmax_scale)
-    batch = cu_seqlens_q.shape[0] - 1
-    group = q.shape[1] // k.shape[1]
-    if q.shape[0] != batch or group > 16:
+    scale = _resolve(q, k.shape, n_heads, kv_heads, head_dim, softmax_scale)
+    q_shape = q.shape
+    if q_shape[0] != cu_seqlens_q.shape[0] - 1 or q_shape[1] // k.shape[1] > 16:
         if k.dtype == torch.float8_e4m3fn:
             raise ValueError("fp8 K/V needs one query per sequence and GQA groups up to 16")
         return inkling_fa4_rel_attention(q, k, v, rel_logits, cu_seqlens_q, cu_seqlens_k,
                                          max_seqlen_q, max_seqlen_k, rel_extent, causal,
                                          window_size, softmax_scale=scale,
                                          return_lse=return_lse, bottom_right=bottom_right)
-    out, lse = _ops().decode(q, k, v, rel_logits, cu_seqlens_q, cu_seqlens_k,
-                             int(max_seqlen_q), int(max_seqlen_k), int(rel_extent), bool(causal),
-                             _window_left(window_size), scale, bool(return_lse),
-                             _flag_bits(bottom_right), float(k_scale), float(v_scale))
+    out, lse = _call("decode", q, k, v, rel_logits, cu_seqlens_q, cu_seqlens_k,
+                     int(max_seqlen_q), int(max_seqlen_k), int(rel_extent), bool(causal),
+                     _window_left(window_size), scale, bool(return_lse),
+                     _flag_bits(bottom_right), float(k_scale), float(v_scale))
     return (out, lse) if return_lse else out
 
 
-@torch.no_grad()
 def inkling_fa4_rel_attention_decode_paged(q, k_cache, v_cache, rel_logits, cu_seqlens_q,
                                            seqused_k, block_table, max_seqlen_q, max_seqlen_k,
                                            rel_extent, causal=True, window_size=(-1, -1), *,
@@ -155,16 +174,14 @@ def inkling_fa4_rel_attention_decode_paged(q, k_cache, v_cache, rel_logits, cu_s
     """
     if k_cache.dim() != 4:
         raise ValueError("k_cache must be [num_blocks, block_size, kv_heads, head_dim]")
-    scale = _resolve(q, k_cache[0], None, None, None, softmax_scale)
-    out, lse = _ops().decode_paged(q, k_cache, v_cache, rel_logits, cu_seqlens_q, seqused_k,
-                                   block_table, int(max_seqlen_q), int(max_seqlen_k),
-                                   int(rel_extent), bool(causal), _window_left(window_size),
-                                   scale, bool(return_lse), _flag_bits(bottom_right),
-                                   float(k_scale), float(v_scale))
+    scale = _resolve(q, k_cache.shape[1:], None, None, None, softmax_scale)
+    out, lse = _call("decode_paged", q, k_cache, v_cache, rel_logits, cu_seqlens_q, seqused_k,
+                     block_table, int(max_seqlen_q), int(max_seqlen_k), int(rel_extent),
+                     bool(causal), _window_left(window_size), scale, bool(return_lse),
+                     _flag_bits(bottom_right), float(k_scale), float(v_scale))
     return (out, lse) if return_lse else out
 
 
-@torch.no_grad()
 def inkling_fa4_rel_attention_rproj(q, k, v, rel_r, rel_w, cu_seqlens_q, cu_seqlens_k,
                                     max_seqlen_q, max_seqlen_k, rel_extent, causal=True,
                                     window_size=(-1, -1), *, softmax_scale=None,
@@ -180,14 +197,14 @@ def inkling_fa4_rel_attention_rproj(q, k, v, rel_r, rel_w, cu_seqlens_q, cu_seql
     r and W split into bf16 hi + lo parts (about 16 significant bits).
     Otherwise as inkling_fa4_rel_attention.
     """
-    scale = _resolve(q, k, None, None, None, softmax_scale)
+    scale = _resolve(q, k.shape, None, None, None, softmax_scale)
     if rel_w.dim() != 2 or rel_w.shape[0] != rel_r.shape[-1]:
         raise ValueError("rel_w must be [d_rel, R'] with d_rel = rel_r.shape[-1]")
     wt = rel_w.t().to(torch.float32).contiguous()  # W^T [R', 16], 64 bytes per distance
-    out, lse = _ops().fwd_rproj(q, k, v, rel_r, wt, cu_seqlens_q, cu_seqlens_k,
-                                int(max_seqlen_q), int(max_seqlen_k), int(rel_extent),
-                                bool(causal), _window_left(window_size), scale, bool(return_lse),
-                                _flag_bits(bottom_right))
+    out, lse = _call("fwd_rproj", q, k, v, rel_r, wt, cu_seqlens_q, cu_seqlens_k,
+                     int(max_seqlen_q), int(max_seqlen_k), int(rel_extent), bool(causal),
+                     _window_left(window_size), scale, bool(return_lse),
+                     _flag_bits(bottom_right))
     return (out, lse) if return_lse else out
 
 
