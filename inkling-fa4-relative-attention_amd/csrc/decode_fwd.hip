@@ -1067,9 +1067,9 @@ __global__ __launch_bounds__(64 * kCombineWaves) void decode_combine_kernel(Deco
   constexpr int kThreads = 64 * kCombineWaves;
   constexpr int kChunks = D / 4 / SPLIT;        // 16-byte chunks of this split
   constexpr int kGroups = kThreads / kChunks;   // part groups
-  __shared__ f32x4_t part_o[kGroups][kChunks];
-  __shared__ float part_m[kGroups];
-  __shared__ float part_l[kGroups];
+  __shared__ f32x4_t part_o[kCombineWaves][kChunks];
+  __shared__ float part_m[kCombineWaves];
+  __shared__ float part_l[kCombineWaves];
   const int head = blockIdx.x;
   const int seq = blockIdx.y;
   const int split = blockIdx.z;
@@ -1119,21 +1119,39 @@ __global__ __launch_bounds__(64 * kCombineWaves) void decode_combine_kernel(Deco
     acc = acc * a_old + a_new * os;
     m = mn;
   }
-  part_o[grp][c] = acc;
-  if (c == 0) {  // every thread of a group has merged the same parts: one m, l
-    part_m[grp] = m;
-    part_l[grp] = l;
+  // The part groups of a wave (64 / kChunks of them, a chunk every kChunks lanes)
+  // meet by lane exchange, the waves in LDS: with every group's partial in LDS, the
+  // walk over up to 64 of them was the longest part of this kernel.
+#pragma unroll
+  for (int off = kChunks; off < 64; off <<= 1) {
+    const float mo = __shfl_xor(m, off), lo = __shfl_xor(l, off);
+    const f32x4_t ao = {__shfl_xor(acc[0], off), __shfl_xor(acc[1], off), __shfl_xor(acc[2], off),
+                        __shfl_xor(acc[3], off)};
+    const float mn = fmaxf(m, mo);
+    const float mu = mn == -INFINITY ? 0.f : mn;
+    const float a_own = fast_exp2(m - mu), a_other = fast_exp2(mo - mu);
+    l = l * a_own + lo * a_other;
+    acc = acc * a_own + ao * a_other;
+    m = mn;
+  }
+  const int wave = tid >> 6;
+  if ((tid & 63) < kChunks) {
+    part_o[wave][c] = acc;
+    if (c == 0) {  // every thread of a wave's first group holds the same m, l
+      part_m[wave] = m;
+      part_l[wave] = l;
+    }
   }
   __syncthreads();
   if (grp != 0) return;
   float mt = part_m[0];
 #pragma unroll
-  for (int g = 1; g < kGroups; ++g) mt = fmaxf(mt, part_m[g]);
+  for (int g = 1; g < kCombineWaves; ++g) mt = fmaxf(mt, part_m[g]);
   const float mu = mt == -INFINITY ? 0.f : mt;
   float lt = 0.f;
   f32x4_t out{};
 #pragma unroll
-  for (int g = 0; g < kGroups; ++g) {
+  for (int g = 0; g < kCombineWaves; ++g) {
     const float a = fast_exp2(part_m[g] - mu);
     lt += a * part_l[g];
     out += a * part_o[g][c];
