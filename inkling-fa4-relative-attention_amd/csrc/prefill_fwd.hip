@@ -1264,7 +1264,13 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
   const int q_step = kPack ? p.q_step : Sh::kBlockQ;  // queries per tile
   // ---- which (q tile, KV chunk, head, sequence): heaviest (last) q tiles first --
   // A q tile's chunks (split KV; one when not splitting) are consecutive, so
-  // a chunk that ends early is followed by the next q tile's work.
+  // a chunk that ends early is followed by the next q tile's work.  The fused
+  // projection, one workgroup per CU, takes the first chunk of every q tile, then
+  // the second, ...: the chunk slots that short q tiles leave empty then come
+  // together, not at every n-th workgroup, where they starved some of an XCD's
+  // shader engines while others ran a second round (2 x 900..2100 tokens 60.6 ->
+  // 51.1 us, 1 x 3000 89.7 -> 77.6; the other kernels, two workgroups per CU, lose:
+  // 1 x 4096 over 4 heads 41.3 -> 48.6).
   int qtile, chunk, head, seq;
   if (p.xcd_spread) {  // ragged (prefill_order)
     const int x = blockIdx.x & 7;
@@ -1287,8 +1293,8 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
     const int per_xcd = p.xcd_pairs;  // pairs per XCD
     const int per_tile = per_xcd * p.tile_group;
     const int qc = slot / per_tile;
-    qtile = p.n_qtiles - 1 - qc / p.n_chunks;
-    chunk = qc % p.n_chunks;
+    qtile = p.n_qtiles - 1 - (kProj ? qc % p.n_qtiles : qc / p.n_chunks);
+    chunk = kProj ? qc / p.n_qtiles : qc % p.n_chunks;
     const int rem = slot % per_tile;
     const int pair = x + 8 * (rem / p.tile_group);
     const int kv_heads = p.tile_heads / p.tile_group;
@@ -1298,8 +1304,8 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
     const int per_tile = p.tile_heads * p.batch;
     const int lin = blockIdx.x;
     const int qc = lin / per_tile;
-    qtile = p.n_qtiles - 1 - qc / p.n_chunks;
-    chunk = qc % p.n_chunks;
+    qtile = p.n_qtiles - 1 - (kProj ? qc % p.n_qtiles : qc / p.n_chunks);
+    chunk = kProj ? qc / p.n_qtiles : qc % p.n_chunks;
     const int rem = lin % per_tile;
     head = rem % p.tile_heads;
     seq = rem / p.tile_heads;

@@ -299,7 +299,7 @@ constexpr SplitRule kPrefillSplitRule = {kPrefillSlots, kPrefillSplitSmallGrid,
 // Fused projection: one 256-row workgroup per CU, and a tile in the bias band costs
 // it about 3 us, so any underfilled grid splits when that saves four tiles.  Whole
 // calls without and with the split (one box, us, Hq 8 / Hkv 2, d 128, extent 1024,
-// bf16 r): 2 x 900..2100 tokens 86.0 -> 60.6, 1 x 1000 66.5 -> 33.2, 1 x 3000 117 -> 90,
+// bf16 r): 2 x 900..2100 tokens 86.0 -> 51.1, 1 x 1000 66.5 -> 32.8, 1 x 3000 117 -> 78,
 // 3 x 100..600 over 300..2000 keys bottom-right 102.5 -> 61.8, 3 x 2000 98.7 -> 93.0
 // (98.0 when 16 tiles had to be saved), 6 x 1200 (240 workgroups, no split) 76.
 constexpr SplitRule kProjSplitRule = {256, 256, 4};
