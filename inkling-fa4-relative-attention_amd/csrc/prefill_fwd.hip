@@ -1479,11 +1479,15 @@ void launch_merge(const PrefillParams& p, hipStream_t stream) {
 // faster (Hq = Hkv = 4: 92.6 -> 72.2 against 75.7; 5 x 500..4000 over 4 heads 83
 // against 88), as with fewer sequences than XCDs to take turns on, and for the
 // KV chunks of a split call (3 x 333..512 tokens over 3K..9K keys: 65.3 against 69.0).
+// Few sequences leave the equal-length order as it was: which of them meets which
+// XCD is then a draw either way (3 x 126..1864 over Hq 16 / Hkv 4 38.2 in it, 42.9
+// in this one; 5 x 409..768 over 4 heads 23.3 against 24.6).
 int64_t prefill_order(PrefillParams& p) {
   const int pairs = p.batch * (p.tile_heads / p.tile_group);
   const int64_t tiles = (int64_t)p.n_qtiles * p.n_chunks;
   p.xcd_spread = 0;
   p.xcd_pairs = pairs % 8 == 0 ? pairs / 8 : 0;
+  if (p.batch < 6) p.ragged = 0;
   if (p.ragged && p.n_chunks == 1) {
     int unit = p.tile_group < 4 ? p.tile_group : 4;
     while (p.tile_group % unit != 0) --unit;

@@ -327,6 +327,9 @@ inline PrefillSplit prefill_split_for(int64_t batch, int64_t n_heads, int64_t ma
   if (chunk <= 0) {
     const int64_t grid = (max_q + block_q - 1) / block_q * n_heads * batch;
     if (grid >= rule.slots || grid > kPrefillSplitMaxGrid) return s;
+    // a short window leaves too few tiles to repay the merge pass (1 x 58..126
+    // queries, window 127, five tiles: 14.3 us split)
+    if (bottom_right && window_left >= 0 && tmax < 8) return s;
     if (grid > rule.small_grid && tmax < kPrefillSplitWideMinTiles) return s;
     const int64_t balanced =
         ((total * batch * n_heads + rule.slots - 1) / rule.slots * kPrefillChunkPct + 99) / 100;
