@@ -222,7 +222,9 @@ int32_t ifa4_prefill_count_tiles(const ifa4_args* args, const int32_t* host_cu_s
  * counts 7/4 of a plain one; ifa4_decode_tile reports the keys per wave of a
  * contiguous 16-bit cache); it writes one (o, lse) partial per (cache, wave)
  * it touches into the workspace.  Pass 2 merges each cache's partials by log-sum-exp and
- * writes out/lse.  The workspace (ifa4_decode_workspace_bytes, 256-byte
+ * writes out/lse.  Calls of short caches or windows (up to 20 steps of 32 keys, more
+ * when the caches are many) take one launch instead, a workgroup per cache, and leave
+ * the workspace untouched.  The workspace (ifa4_decode_workspace_bytes, 256-byte
  * aligned, contents on entry irrelevant) is scratch for one call; calls that
  * share a workspace must not overlap.  Replaces
  * inkling_fa4_rel_attention_decode_triton
