@@ -4,7 +4,7 @@ the order runs each query tile exactly once.
 The order depends on heads per kv head, kv heads and batch: units of up to four
 heads whose query tiles go round 8, 4, 2 or 1 XCDs (8 / 1 .. 64 / 8 heads, with
 batches that are and are not multiples of the XCDs), and the linear order
-(one head per kv head, head counts that do not divide 8, few sequences).  A tile
+(one head per kv head, head counts that do not divide 8, under six sequences).  A tile
 left out shows as rows that were never written, one run twice is harmless, a wrong
 (sequence, head) as wrong rows: outputs against the fp32 oracle, 16-bit rounding
 of P and of the output (2e-2) and the fp32 LSE (1e-3) as in the other prefill tests.
@@ -17,10 +17,10 @@ from oracle import ref_rel_attn_with_lse
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("hq,hkv,batch", [(4, 1, 8), (8, 2, 9), (8, 2, 4), (8, 2, 3), (8, 1, 5),
-                                          (16, 4, 5), (32, 4, 2), (64, 16, 3), (64, 8, 2),
-                                          (6, 3, 5), (8, 4, 6), (12, 2, 4), (10, 2, 3), (4, 4, 5),
-                                          (8, 8, 3)])
+@pytest.mark.parametrize("hq,hkv,batch", [(4, 1, 8), (8, 2, 9), (8, 2, 8), (8, 2, 5), (8, 1, 7),
+                                          (16, 4, 7), (32, 4, 6), (64, 16, 6), (64, 8, 7),
+                                          (6, 3, 7), (8, 4, 6), (12, 2, 6), (10, 2, 7), (4, 4, 8),
+                                          (8, 8, 9)])
 def test_ragged_order_runs_every_tile(cuda, hq, hkv, batch):
     lens = [300, 33, 1, 129, 0, 257, 128, 64, 190][:batch]
     case = testing.make_case("order", lens, lens, hq, hkv, 64, torch.bfloat16, seed=hq + batch,
