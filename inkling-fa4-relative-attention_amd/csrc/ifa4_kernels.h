@@ -6,6 +6,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "workgroup_order.h"
+
 struct ifa4_args;
 
 namespace ifa4 {
@@ -34,11 +36,7 @@ struct PrefillParams {
   int32_t rel_dtype;    // 0 bf16, 1 fp16, 2 fp32
   int32_t n_qtiles;     // ceil(max_seqlen_q / block_q)
   int32_t ragged;       // 1: sequences well shorter than the longest (rows against batch * max)
-  int32_t xcd_pairs;    // (sequence, kv head) pairs per XCD in the XCD-aware order, or 0
-  // Order of a ragged call (xcd_spread > 0): xcd_unit query heads of one kv head
-  // run together on one XCD, the query tiles of such a unit go round xcd_spread
-  // XCDs (a power of two), and an XCD serves xcd_heads units of a sequence.
-  int32_t xcd_spread, xcd_unit, xcd_heads;
+  WorkgroupOrder order; // set by launch_prefill
   float scale_log2;     // softmax_scale * log2(e)
   // Split KV (chunk_tiles > 0): each q tile's KV tile range is cut into chunks
   // of chunk_tiles tiles, one workgroup each (n_chunks chunk slots per q tile in

@@ -50,7 +50,7 @@
 // is served from one XCD's L2 (measured: 72 instead of 337 MiB fetched from
 // the fabric per call on the 8 x 4096 workload).  Heaviest q tiles go first.
 // Sequences of unequal length would load the XCDs unequally that way (the
-// busiest XCD set the time of a ragged batch); their order is in prefill_order.
+// busiest XCD set the time of a ragged batch); their order is in workgroup_order.
 //
 // Tile classes per (wave, KV tile): fully masked -> skipped (causal: keys after
 // the wave's last row; window: keys left of the window); edge (diagonal, window
@@ -1271,49 +1271,18 @@ __global__ __launch_bounds__(Sh::kThreads) __attribute__((amdgpu_waves_per_eu(
   // shader engines while others ran a second round (2 x 900..2100 tokens 60.6 ->
   // 51.1 us, 1 x 3000 89.7 -> 77.6; the other kernels, two workgroups per CU, lose:
   // 1 x 4096 over 4 heads 41.3 -> 48.6).
-  int qtile, chunk, head, seq;
-  if (p.xcd_spread) {  // ragged (prefill_order)
-    const int x = blockIdx.x & 7;
-    int slot = blockIdx.x >> 3;
-    const int m = slot % p.xcd_unit;
-    slot /= p.xcd_unit;
-    const int k = slot % p.xcd_heads;
-    slot /= p.xcd_heads;
-    const int rounds = (p.batch + p.xcd_spread - 1) / p.xcd_spread;
-    const int qc = slot / rounds;
-    seq = (slot + qc) % rounds * p.xcd_spread + ((x + 7 * qc) & (p.xcd_spread - 1));
-    if (seq >= p.batch) return;
-    head = (p.xcd_spread > 1 ? x / p.xcd_spread : x * p.xcd_heads + k) * p.xcd_unit + m;
-    qtile = p.n_qtiles - 1 - qc / p.n_chunks;
-    chunk = qc % p.n_chunks;
-  } else if (p.xcd_pairs) {
-    // Workgroup i runs on XCD i % 8.  Give XCD x the (sequence, kv head) pairs
-    // x, x+8, ... so their K/V stay in that XCD's L2; heaviest q tiles first.
-    const int x = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    const int per_xcd = p.xcd_pairs;  // pairs per XCD
-    const int per_tile = per_xcd * p.tile_group;
-    const int qc = slot / per_tile;
-    qtile = p.n_qtiles - 1 - (kProj ? qc % p.n_qtiles : qc / p.n_chunks);
-    chunk = kProj ? qc / p.n_qtiles : qc % p.n_chunks;
-    const int rem = slot % per_tile;
-    const int pair = x + 8 * (rem / p.tile_group);
-    const int kv_heads = p.tile_heads / p.tile_group;
-    seq = pair / kv_heads;
-    head = (pair % kv_heads) * p.tile_group + rem % p.tile_group;
-  } else {
-    const int per_tile = p.tile_heads * p.batch;
-    const int lin = blockIdx.x;
-    const int qc = lin / per_tile;
-    qtile = p.n_qtiles - 1 - (kProj ? qc % p.n_qtiles : qc / p.n_chunks);
-    chunk = kProj ? qc / p.n_qtiles : qc % p.n_chunks;
-    const int rem = lin % per_tile;
-    head = rem % p.tile_heads;
-    seq = rem / p.tile_heads;
-    if (p.ragged) seq = (seq + qc) % p.batch;
+  WorkgroupPlace at;
+  if (!workgroup_place(p.order, blockIdx.x, p.batch, &at)) return;
+  int qtile = at.qc, chunk = 0;
+  if (p.n_chunks > 1) {
+    qtile = kProj ? at.qc % p.n_qtiles : at.qc / p.n_chunks;
+    chunk = kProj ? at.qc / p.n_qtiles : at.qc % p.n_chunks;
   }
+  qtile = p.n_qtiles - 1 - qtile;
+  const int head = at.head;
 
   WorkItem it;
-  set_sequence(p, it, seq);
+  set_sequence(p, it, at.seq);
   it.q0 = qtile * q_step;
   if (it.q0 >= it.lq) return;
   it.q_end = min(it.q0 + q_step, it.lq);
@@ -1464,51 +1433,13 @@ void launch_merge(const PrefillParams& p, hipStream_t stream) {
                      0, stream, p);
 }
 
-// Workgroup order and grid of a call.  Pairs in fixed XCDs suit equal lengths
-// (every pair the same work).  In a ragged batch the work differs by sequence
-// but not by head, so heads go to XCDs instead, and a sequence's query tiles
-// take turns on the XCDs of its heads: units of up to four heads of one kv head
-// stay together (their K/V tiles come from HBM once), unit v of a sequence on
-// XCDs v * spread .. + spread - 1.  Against pairs in fixed XCDs (one box, us;
-// per-token bf16 bias of extent 1024 unless said): 16 x 17..1900 tokens,
-// Hq 8 / Hkv 2 133.5 -> 93, shared table 93.9 -> 61.8, Hq 16 / Hkv 4 197 -> 183,
-// Hq 8 / Hkv 1 171 -> 92; 12 x 1000..4096, shared table 249 -> 206.  Units of one
-// head 136 and of two 100 on the first; one head of every kv head per XCD (the
-// linear order) 100.  With one head per kv head there is no K/V to share, and
-// the linear order, its sequences turned by one per query tile, is as fast or
-// faster (Hq = Hkv = 4: 92.6 -> 72.2 against 75.7; 5 x 500..4000 over 4 heads 83
-// against 88), as with fewer sequences than XCDs to take turns on, and for the
-// KV chunks of a split call (3 x 333..512 tokens over 3K..9K keys: 65.3 against 69.0).
-// Few sequences leave the equal-length order as it was: which of them meets which
-// XCD is then a draw either way (3 x 126..1864 over Hq 16 / Hkv 4 38.2 in it, 42.9
-// in this one; 5 x 409..768 over 4 heads 23.3 against 24.6).
-int64_t prefill_order(PrefillParams& p) {
-  const int pairs = p.batch * (p.tile_heads / p.tile_group);
-  const int64_t tiles = (int64_t)p.n_qtiles * p.n_chunks;
-  p.xcd_spread = 0;
-  p.xcd_pairs = pairs % 8 == 0 ? pairs / 8 : 0;
-  if (p.batch < 6) p.ragged = 0;
-  if (p.ragged && p.n_chunks == 1) {
-    int unit = p.tile_group < 4 ? p.tile_group : 4;
-    while (p.tile_group % unit != 0) --unit;
-    const int units = p.tile_heads / unit;  // per sequence
-    const int spread = units % 8 == 0 ? 1 : 8 % units == 0 ? 8 / units : 0;
-    if (unit > 1 && spread > 0 && p.batch >= spread) {
-      p.xcd_unit = unit;
-      p.xcd_spread = spread;
-      p.xcd_heads = spread > 1 ? 1 : units / 8;
-      return tiles * ((p.batch + spread - 1) / spread) * p.xcd_heads * unit * 8;
-    }
-    p.xcd_pairs = 0;
-  }
-  return tiles * p.tile_heads * p.batch;
-}
-
 template <typename Sh, int D, typename Tag, typename Rel, bool kProj, bool kTab, bool kPack>
 hipError_t launch_prefill_t(const PrefillParams& p_in, hipStream_t stream) {
   PrefillParams p = p_in;
   if (p.n_chunks < 1) p.n_chunks = 1;
-  const int64_t blocks = prefill_order(p);
+  p.order =
+      workgroup_order(p.tile_heads, p.tile_group, p.batch, p.ragged != 0, p.n_chunks);
+  const int64_t blocks = order_blocks(p.order) * p.n_qtiles * p.n_chunks;
   if (blocks <= 0) return hipSuccess;
   hipLaunchKernelGGL((prefill_fwd_kernel<Sh, D, Tag, Rel, kProj, kTab, kPack>), dim3((unsigned)blocks),
                      dim3(Sh::kThreads), 0, stream, p);
