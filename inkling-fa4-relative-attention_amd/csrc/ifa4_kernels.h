@@ -35,7 +35,7 @@ struct PrefillParams {
   int32_t no_prune;
   int32_t rel_dtype;    // 0 bf16, 1 fp16, 2 fp32
   int32_t n_qtiles;     // ceil(max_seqlen_q / block_q)
-  int32_t ragged;       // 1: sequences well shorter than the longest (rows against batch * max)
+  int32_t ragged;       // rows a sixteenth (1) or a quarter (2) below batch * longest, or 0
   WorkgroupOrder order; // set by launch_prefill
   float scale_log2;     // softmax_scale * log2(e)
   // Split KV (chunk_tiles > 0): each q tile's KV tile range is cut into chunks

@@ -78,37 +78,42 @@ inline int64_t order_blocks(const WorkgroupOrder& o) {
   return (int64_t)o.unit * o.rounds << o.lanes;
 }
 
-// The order of a call.  Pairs in fixed XCDs suit equal lengths
-// (every pair the same work).  In a ragged batch the work differs by sequence
-// but not by head, so heads go to XCDs instead, and a sequence's query tiles
-// take turns on the XCDs of its heads: units of up to four heads of one kv head
-// stay together (their K/V tiles come from HBM once), unit v of a sequence on
-// XCDs v * spread .. + spread - 1.  Against pairs in fixed XCDs (one box, us;
-// per-token bf16 bias of extent 1024 unless said): 16 x 17..1900 tokens,
-// Hq 8 / Hkv 2 133.5 -> 93, shared table 93.9 -> 61.8, Hq 16 / Hkv 4 197 -> 183,
-// Hq 8 / Hkv 1 171 -> 92; 12 x 1000..4096, shared table 249 -> 206.  Units of one
-// head 136 and of two 100 on the first; one head of every kv head per XCD (the
-// linear order) 100.  With one head per kv head there is no K/V to share, and
-// the linear order, its sequences turned by one per query tile, is as fast or
-// faster (Hq = Hkv = 4: 92.6 -> 72.2 against 75.7; 5 x 500..4000 over 4 heads 83
-// against 88), as with fewer sequences than XCDs to take turns on, and for the
-// KV chunks of a split call (3 x 333..512 tokens over 3K..9K keys: 65.3 against 69.0).
-// Few sequences leave the equal-length order as it was: which of them meets which
-// XCD is then a draw either way (3 x 126..1864 over Hq 16 / Hkv 4 38.2 in it, 42.9
-// in this one; 5 x 409..768 over 4 heads 23.3 against 24.6).
-inline WorkgroupOrder workgroup_order(int32_t heads, int32_t group, int32_t batch, bool ragged,
-                                      int32_t chunks) {
+// The order of a call.  Pairs suit equal lengths: every pair is the same work.  In a
+// ragged batch (`ragged` 1: rows a sixteenth below batch times the longest, 2: a
+// quarter) of more work than the chip holds at once (`live` workgroups with work,
+// estimated from the rows, against `slots` resident ones) the busiest XCD sets the
+// time, and work differs by sequence but not by head: heads go to XCDs then.  Units
+// of four heads of one kv head (their K/V tiles come from HBM once) in the spread
+// order; smaller groups in the linear order with its sequences turned, in the place
+// of pairs.  (One box, us, before -> after; per-token bf16 bias of extent 1024
+// unless said; `proj`: the fused projection.)
+//   spread  16 x 17..1900 tokens, Hq 8 / Hkv 2 134 -> 95, shared table 93.9 -> 61.8,
+//           Hq 16 / Hkv 4 201 -> 186, Hq 8 / Hkv 1 171 -> 95; 12 x 500..1500, 8 / 2 74.8 ->
+//           61.0; 8 x 100..1500 not causal 95.0 -> 65.6, causal 58.2 -> 57.4; proj 16 x
+//           17..1900 122.8 -> 94.2, 24 x 50..800 60.1 -> 52.4
+//   turned  16 x 17..1900, Hq = Hkv = 4 93.3 -> 73.5, 6 / 3 97.5 -> 82.3, 8 / 4 134.7 ->
+//           104.7 (spread in units of two: 118.9); proj 8 / 4 8 x 500..3000 144 -> 115
+// What keeps the order of equal lengths, with what it would measure otherwise:
+// workgroups all resident at once (spread 6 x 300..2000, 8 / 2, 456 live 61.9 -> 62.2,
+// 9 x 50..1200, 392 40.5 -> 43.2; turned 16 x 100..700, 6 / 3, 395 28.4 -> 31.4; proj 10 x
+// 100..600, 16 / 4, 256 of 256 40.6 -> 43.2, hence a quarter more there); the turned
+// order, and the projection, of lengths less than a quarter apart (32 x 400..520, 4 / 4
+// 30.4 -> 31.5); the linear order, taken where pairs do not divide evenly, is not
+// turned (12 x 500..1500, 6 / 3 61.0 -> 63.8); split calls (chunks > 1: 3 x 333..512 tokens
+// over 3K..9K keys 65.3 -> 69.0).
+inline WorkgroupOrder workgroup_order(int32_t heads, int32_t group, int32_t batch, int32_t ragged,
+                                      int32_t chunks, int64_t live, int64_t slots, bool proj) {
   const bool pairs = (int64_t)batch * (heads / group) % 8 == 0;
-  const bool turn = ragged && batch >= 6;
-  if (turn && chunks == 1) {
+  if (ragged > 0 && batch >= 6 && chunks == 1 && live >= (proj ? slots + slots / 4 : slots)) {
     int32_t unit = group < 4 ? group : 4;
     while (group % unit != 0) --unit;
     const int32_t units = heads / unit;
     const int32_t xcds = units % 8 == 0 ? 1 : 8 % units == 0 ? 8 / units : 0;
-    if (unit > 1 && xcds > 0 && batch >= xcds) return spread_order(heads, unit, batch);
-    return linear_order(heads, batch, true);
+    if (unit == 4 && xcds > 0 && batch >= xcds && ragged > (proj ? 1 : 0))
+      return spread_order(heads, unit, batch);
+    if (pairs && ragged > 1) return linear_order(heads, batch, true);
   }
-  return pairs ? pairs_order(heads, group, batch) : linear_order(heads, batch, turn);
+  return pairs ? pairs_order(heads, group, batch) : linear_order(heads, batch, false);
 }
 
 }  // namespace ifa4
