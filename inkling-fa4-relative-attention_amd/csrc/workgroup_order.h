@@ -96,22 +96,24 @@ inline int64_t order_blocks(const WorkgroupOrder& o) {
 // What keeps the order of equal lengths, with what it would measure otherwise:
 // workgroups all resident at once (spread 6 x 300..2000, 8 / 2, 456 live 61.9 -> 62.2,
 // 9 x 50..1200, 392 40.5 -> 43.2; turned 16 x 100..700, 6 / 3, 395 28.4 -> 31.4; proj 10 x
-// 100..600, 16 / 4, 256 of 256 40.6 -> 43.2, hence a quarter more there); the turned
+// 100..600, 16 / 4, 256 of 256 40.6 -> 43.2, hence a quarter more there); sequences of one
+// query tile, which has no turn to take (64 x 45..90 queries over 1K..2K keys, 16 / 2
+// 136.2 -> 139.4); groups above two in the turned order, whose heads then meet their K/V
+// in several L2s (the same, 24 / 4 208 -> 233; 200 x over 150..300, 6 / 2 58.1 -> 60.6); the turned
 // order, and the projection, of lengths less than a quarter apart (32 x 400..520, 4 / 4
 // 30.4 -> 31.5); the linear order, taken where pairs do not divide evenly, is not
 // turned (12 x 500..1500, 6 / 3 61.0 -> 63.8); split calls (chunks > 1: 3 x 333..512 tokens
 // over 3K..9K keys 65.3 -> 69.0).
 inline WorkgroupOrder workgroup_order(int32_t heads, int32_t group, int32_t batch, int32_t ragged,
-                                      int32_t chunks, int64_t live, int64_t slots, bool proj) {
+                                      int32_t qtiles, int32_t chunks, int64_t live, int64_t slots,
+                                      bool proj) {
   const bool pairs = (int64_t)batch * (heads / group) % 8 == 0;
-  if (ragged > 0 && batch >= 6 && chunks == 1 && live >= (proj ? slots + slots / 4 : slots)) {
-    int32_t unit = group < 4 ? group : 4;
-    while (group % unit != 0) --unit;
-    const int32_t units = heads / unit;
-    const int32_t xcds = units % 8 == 0 ? 1 : 8 % units == 0 ? 8 / units : 0;
-    if (unit == 4 && xcds > 0 && batch >= xcds && ragged > (proj ? 1 : 0))
-      return spread_order(heads, unit, batch);
-    if (pairs && ragged > 1) return linear_order(heads, batch, true);
+  if (ragged > 0 && batch >= 6 && qtiles > 1 && chunks == 1 &&
+      live >= (proj ? slots + slots / 4 : slots)) {
+    const int32_t units = group % 4 == 0 ? heads / 4 : 0;
+    const int32_t xcds = units == 0 ? 0 : units % 8 == 0 ? 1 : 8 % units == 0 ? 8 / units : 0;
+    if (xcds > 0 && batch >= xcds && ragged > (proj ? 1 : 0)) return spread_order(heads, 4, batch);
+    if (pairs && ragged > 1 && group <= 2) return linear_order(heads, batch, true);
   }
   return pairs ? pairs_order(heads, group, batch) : linear_order(heads, batch, false);
 }

@@ -19,7 +19,8 @@ using namespace ifa4;
 // 0 when the workgroups of the call take every place exactly once
 extern "C" int check(int heads, int group, int batch, int ragged, int chunks, long live,
                      long slots, int proj, int qtiles, int* form) {
-  const WorkgroupOrder o = workgroup_order(heads, group, batch, ragged, chunks, live, slots, proj);
+  const WorkgroupOrder o = workgroup_order(heads, group, batch, ragged, qtiles, chunks, live,
+                                           slots, proj);
   form[0] = o.lanes;
   form[1] = o.pair_heads;
   form[2] = o.lanes && !o.pair_heads ? 1 << o.spread_log : 0;
@@ -91,6 +92,8 @@ def test_every_place_once(lib):
     (8, 4, 16, dict(live=440, slots=256, proj=1), dict(lanes=3, xcds=4, turn=1)),
     (8, 2, 16, dict(live=440, slots=256, proj=1), dict(lanes=0, turn=1)),
     (8, 4, 16, dict(live=440, slots=256, proj=1, ragged=1), dict(lanes=3, pair_heads=2)),
+    (8, 4, 64, dict(live=600, qtiles=1), dict(lanes=3, pair_heads=2)),
+    (24, 6, 64, dict(live=5000), dict(lanes=3, pair_heads=4)),
     (16, 4, 10, dict(live=319, slots=256, proj=1), dict(lanes=3, pair_heads=4)),
     (4, 4, 12, dict(live=600), dict(lanes=3, xcds=8, turn=1)),
     (4, 4, 7, dict(live=600), dict(lanes=0, turn=0)),          # fewer sequences than XCDs
