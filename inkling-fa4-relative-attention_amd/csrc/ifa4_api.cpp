@@ -194,24 +194,37 @@ ifa4::PrefillParams make_prefill_params(const ifa4_args* a) {
 }
 
 // Query heads of a kv head whose rows share the query tiles: the whole group
-// when that takes fewer tiles (prefill_packs), and its q rows and bias rows stay
+// when that takes fewer tiles (prefill_can_pack), the call gains by it (prefill_packs;
+// IFA4_FLAG_SPLIT_KV_2 packs without asking), and its q rows and bias rows stay
 // below the 2 GiB of a buffer resource (a shared bias table: its copies below
 // the LDS they get); else one.
 int prefill_pack(const ifa4_args* a) {
   const int64_t kLimit = int64_t(1) << 31;
   const int64_t group = a->n_heads / a->kv_heads;
   const int bq = ifa4::prefill_block_q();
-  if (!ifa4::prefill_packs(group, a->max_seqlen_q, bq)) return 1;
+  if (!ifa4::prefill_can_pack(group, a->max_seqlen_q, bq)) return 1;
+  ifa4::PrefillParams p{};
+  p.rel_st = a->rel_stride_t;
+  p.rel_extent = a->rel_extent;
+  const bool table = ifa4::prefill_tab(p);
+  if ((a->flags & IFA4_FLAG_SPLIT_KV_2) == 0) {
+    int64_t key_tiles, total;
+    ifa4::prefill_tile_work(
+        a->max_seqlen_q, a->max_seqlen_k,
+        ifa4::plan_masks(a->causal != 0, a->window_left, (a->flags & IFA4_FLAG_BOTTOM_RIGHT) != 0,
+                         a->max_seqlen_q, a->max_seqlen_k),
+        bq, ifa4::prefill_block_k(), &key_tiles, &total);
+    if (!ifa4::prefill_packs((int64_t)a->batch * a->n_heads, key_tiles, group, a->max_seqlen_q,
+                             table))
+      return 1;
+  }
   const int64_t rows = (int64_t)a->max_seqlen_q + bq;
   const int64_t esize = a->rel_dtype == IFA4_FP32 ? 4 : 2;
   if ((rows * a->q_stride_t + (group - 1) * a->q_stride_h + a->head_dim) * 2 >= kLimit) return 1;
   if (a->rel_extent > 0 &&
       (rows * a->rel_stride_t + (group - 1) * a->rel_stride_h + a->rel_width) * esize >= kLimit)
     return 1;
-  ifa4::PrefillParams p{};
-  p.rel_st = a->rel_stride_t;
-  p.rel_extent = a->rel_extent;
-  if (ifa4::prefill_tab(p) && !ifa4::prefill_tab_packs(a->rel_extent, (int)group)) return 1;
+  if (table && !ifa4::prefill_tab_packs(a->rel_extent, (int)group)) return 1;
   return (int)group;
 }
 

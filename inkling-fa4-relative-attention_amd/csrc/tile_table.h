@@ -224,22 +224,6 @@ constexpr int64_t kPrefillChunkPct = IFA4_PREFILL_CHUNK_PCT;
 #endif
 constexpr int64_t kPrefillSplitWideMinTiles = 16;
 
-// Packed rows: the query heads of a kv head share query tiles (block_q / group
-// queries x group heads) when every sequence fits one tile of block_q queries and
-// packing leaves at most three quarters of the tiles.  A sequence of a few
-// queries otherwise takes one workgroup per head with one or two of its four
-// waves at work, each streaming the same K/V.  With it against without (one box,
-// us, Hq 8 / Hkv 2, d 128): 12 x 2..5 queries over 1K..8K keys 42.4 -> 22.9, 24 x
-// 2..8 91.6 -> 41.3, Hq 8 / Hkv 1 56.5 -> 24.6, 3 x 20..40 over 3K..9K 26.8 -> 22.4,
-// x 50..96 31.3 -> 29.2.  Past a tile per head it no longer pays on every call:
-// 3 x 120..200 45 -> 39, but 333..410 64 -> 69, 16 x 17..300 without a cache
-// 15.5 -> 18.8 (fewer, fuller workgroups leave CUs idle).
-inline bool prefill_packs(int64_t group, int64_t max_q, int64_t block_q) {
-  if (group <= 1 || group > block_q || max_q <= 0 || max_q > block_q) return false;
-  const int64_t step = block_q / group;
-  return 4 * ((max_q + step - 1) / step) <= 3 * group;
-}
-
 struct PrefillSplit {
   int32_t chunk_tiles;  // 0: no split
   int32_t n_chunks;     // chunk slots per query tile in the grid
@@ -252,11 +236,56 @@ struct PrefillMasks {
   int64_t window_left;  // -1: none
   int64_t qpos;
 };
+// The masks a plan goes by.  It takes the longest cache for every sequence and,
+// bottom-right without a window, every key for every query (the causal mask takes max_q
+// keys at most).
+inline PrefillMasks plan_masks(bool causal, int64_t window_left, bool bottom_right, int64_t max_q,
+                               int64_t max_k) {
+  return PrefillMasks{causal && !(bottom_right && window_left < 0), window_left,
+                      bottom_right && max_k > max_q ? max_k - max_q : int64_t(0)};
+}
 // Keys [kbeg, kend) that queries [q0, q_hi) of a sequence over lk keys see.
 inline void prefill_keys(int64_t q0, int64_t q_hi, int64_t lk, const PrefillMasks& m,
                          int64_t* kbeg, int64_t* kend) {
   *kend = m.causal && q_hi + m.qpos < lk ? q_hi + m.qpos : lk;
   *kbeg = m.window_left >= 0 && q0 + m.qpos > m.window_left ? q0 + m.qpos - m.window_left : 0;
+}
+
+// Packed rows: the query heads of a kv head share query tiles (block_q / group
+// queries x group heads) when every sequence fits one tile of block_q queries and
+// packing leaves at most three quarters of the tiles.  A sequence of a few
+// queries otherwise takes one workgroup per head with one or two of its four
+// waves at work, each streaming the same K/V.
+inline bool prefill_can_pack(int64_t group, int64_t max_q, int64_t block_q) {
+  if (group <= 1 || group > block_q || max_q <= 0 || max_q > block_q) return false;
+  const int64_t step = block_q / group;
+  return 4 * ((max_q + step - 1) / step) <= 3 * group;
+}
+
+// It pays where the call has more work than it has room for (grid: workgroups without
+// it, key_tiles: of the longest range): a call whose workgroups are all resident at
+// once and short is one range long either way, and packed rows fill that range's
+// waves or cut it into chunks and a merge pass.  So it packs
+//   - more workgroups than fit at once: 200 x 8 queries 20.8 -> 7.4 us, x 64 26.0 -> 21.3,
+//     64 x 17..96 over Hq 16 / Hkv 2 21.2 -> 19.7;
+//   - ranges of 16 tiles on, where half of the 32-row waves go (12 x 2..5 queries over
+//     1K..8K keys 42.4 -> 22.9, 4 x 16 over 14K 31.6 -> 22.6), or the ranges together
+//     are 6000 tiles of up to 32 queries, or of any if they are 64 on (16 x 32 over 8K
+//     64.3 -> 46.1, 64 x 24 over 2K 57.3 -> 43.1, 4 x 64 over 14K 41.6 -> 34.8);
+//   - where three quarters of the waves go and the bias is per token: 64 x 2 over 500
+//     keys 17.5 -> 14.3 (shared table, whose tiles are cheap, x 8 14.3 -> 15.9).
+// Without one of these it measured (packed against not): 64 x 32 over 500 keys 20.4 ->
+// 25.9, 64 x 96 28.9 -> 32.4, 64 x 64 over 2K 71.1 -> 73.5, 16 x 24 without a cache 6.6 ->
+// 7.1, 64 x 17..96 12.4 -> 13.5 (shared table 10.9 -> 13.3), 4 x 64 over 4K 23.2 -> 26.2.
+// (One box, Hq 8 / Hkv 2, d 128, per-token bf16 bias unless said.)
+inline bool prefill_packs(int64_t grid, int64_t key_tiles, int64_t group, int64_t max_q,
+                          bool table) {
+  const int64_t waves = group * ((max_q + 31) / 32), packed = (max_q * group + 31) / 32;
+  if (grid > kPrefillSlots) return true;
+  if (key_tiles >= 16 &&
+      (2 * packed <= waves || (grid * key_tiles >= 6000 && (max_q <= 32 || key_tiles >= 64))))
+    return true;
+  return !table && 4 * packed <= waves && grid * key_tiles >= 512;
 }
 
 // Tiles of the longest query tile and of all query tiles of one (sequence,
@@ -319,8 +348,7 @@ inline PrefillSplit prefill_split_for(int64_t batch, int64_t n_heads, int64_t ma
                                       const SplitRule& rule = kPrefillSplitRule) {
   PrefillSplit s{0, 1, 1};
   if (batch <= 0 || max_q <= 0 || max_k <= 0) return s;
-  const PrefillMasks masks{causal && !(bottom_right && window_left < 0), window_left,
-                           bottom_right && max_k > max_q ? max_k - max_q : int64_t(0)};
+  const PrefillMasks masks = plan_masks(causal, window_left, bottom_right, max_q, max_k);
   int64_t tmax = 0, total = 0;
   prefill_tile_work(max_q, max_k, masks, block_q, block_k, &tmax, &total);
   int64_t chunk = forced_chunk;

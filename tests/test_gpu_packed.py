@@ -1,11 +1,12 @@
 """Prefill calls of a few queries per sequence over a cache: packed rows (the
 query heads of a kv head share query tiles) and the merge of many chunks.
 
-Packed rows start at 96 queries for groups of four (three quarters of the tiles);
-sizes sit on both sides of that, at tile edges and with groups that do not divide
-the 128 rows (3, 6, 12).  Everything is compared with the fp32 oracle (16-bit
-rounding of P and of the output: 2e-2; fp32 LSE: 1e-3), and pruned with unpruned
-launches bit for bit.
+Rows pack up to 96 queries for groups of four (three quarters of the tiles); sizes sit
+on both sides of that, at tile edges and with groups that do not divide the 128 rows
+(3, 6, 12).  Within that a call packs by its work (the host test has both sides), and
+always under the test flag of two-tile chunks, so every case runs both ways.
+Everything is compared with the fp32 oracle (16-bit rounding of P and of the output:
+2e-2; fp32 LSE: 1e-3), and pruned with unpruned launches bit for bit.
 """
 import pytest
 import torch
@@ -24,20 +25,51 @@ def _check(case, dev, bottom_right=True):
     print(f"{case.name}: q {tuple(case.q.shape)}, k {tuple(case.k.shape)}, causal {case.causal}, "
           f"window {case.window_left}, bottom-right {bottom_right}", flush=True)
     c = case.to(dev)
-    out, lse = _run(c, 0, bottom_right)
     want_out, want_lse = ref_rel_attn_with_lse(
         case.q, case.k, case.v, case.rel, case.cu_q, case.cu_k, case.scale, case.rel_extent,
         causal=case.causal, window_left=case.window_or_none, bottom_right=bottom_right)
     rows = ~torch.isnan(want_out).any(-1)  # rows with a visible key
-    out, lse = out.cpu(), lse.cpu()
-    torch.testing.assert_close(out.float()[rows], want_out.float()[rows], atol=2e-2, rtol=2e-2)
-    torch.testing.assert_close(lse.T[rows], want_lse.T[rows], atol=1e-3, rtol=0)
-    assert bool((out[~rows] == 0).all()) and bool((lse.T[~rows] == float("-inf")).all())
-    full = _run(c, _abi.IFA4_FLAG_NO_PRUNE, bottom_right)
-    assert torch.equal(full[0].cpu(), out) and torch.equal(full[1].cpu(), lse)
-    two, lse2 = _run(c, _abi.IFA4_FLAG_SPLIT_KV_2, bottom_right)
-    torch.testing.assert_close(lse2.cpu(), lse, atol=1e-4, rtol=0)
-    torch.testing.assert_close(two.float().cpu(), out.float(), atol=2e-2, rtol=2e-2)
+    runs = []
+    for flags in (0, _abi.IFA4_FLAG_SPLIT_KV_2):
+        out, lse = (x.cpu() for x in _run(c, flags, bottom_right))
+        torch.testing.assert_close(out.float()[rows], want_out.float()[rows], atol=2e-2, rtol=2e-2)
+        torch.testing.assert_close(lse.T[rows], want_lse.T[rows], atol=1e-3, rtol=0)
+        assert bool((out[~rows] == 0).all()) and bool((lse.T[~rows] == float("-inf")).all())
+        full = _run(c, flags | _abi.IFA4_FLAG_NO_PRUNE, bottom_right)
+        assert torch.equal(full[0].cpu(), out) and torch.equal(full[1].cpu(), lse)
+        runs.append((out, lse))
+    torch.testing.assert_close(runs[1][1], runs[0][1], atol=1e-4, rtol=0)
+    torch.testing.assert_close(runs[1][0].float(), runs[0][0].float(), atol=2e-2, rtol=2e-2)
+
+
+def _workspace(batch, q, keys, hq, hkv, d=128, **kw):
+    """Workspace of a bottom-right call, and the chunk slots it holds."""
+    fields = dict(q=1 << 20, k=1 << 20, v=1 << 20, out=1 << 20, cu_seqlens_q=1 << 20,
+                  cu_seqlens_k=1 << 20, rel=1 << 20, q_stride_t=hq * d, q_stride_h=d,
+                  k_stride_t=hkv * d, k_stride_h=d, v_stride_t=hkv * d, v_stride_h=d,
+                  out_stride_t=hq * d, out_stride_h=d, rel_stride_t=hq * 1024, rel_stride_h=1024,
+                  total_q=batch * q, total_k=batch * keys, batch=batch, n_heads=hq, kv_heads=hkv,
+                  head_dim=d, rel_extent=1024, rel_width=1024, max_seqlen_q=q, max_seqlen_k=keys,
+                  causal=1, flags=_abi.IFA4_FLAG_BOTTOM_RIGHT, qkv_dtype=_abi.IFA4_BF16,
+                  rel_dtype=_abi.IFA4_BF16)
+    fields.update(kw)
+    n = _abi.lib().ifa4_prefill_workspace_bytes(_abi.make_args(**fields))
+    return n // (hq * batch * q * (d + 1) * 4)
+
+
+# chunk slots of the plan without packed rows (per head) and with them, and which of
+# the two the call takes: packed rows only where they were measured to pay
+@pytest.mark.parametrize("batch,q,keys,hq,hkv,slots", [
+    (64, 32, 532, 8, 2, 0),      # 512 workgroups of nine tiles, resident at once
+    (64, 96, 596, 8, 2, 0),
+    (16, 24, 24, 8, 2, 0),       # prompts without a cache
+    (4, 64, 4064, 8, 2, 16),     # 32 workgroups in chunks of four tiles (packed: two, 32 slots)
+    (12, 5, 8005, 8, 2, 21),     # packed: 24 workgroups in chunks of six (unpacked: 25, six)
+    (64, 24, 2024, 8, 2, 4),     # packed: 128 in chunks of eight (unpacked: not split)
+    (16, 32, 8032, 8, 2, 16),    # packed: 32 workgroups in chunks of eight (unpacked: four slots)
+])
+def test_packed_where_it_pays(batch, q, keys, hq, hkv, slots):
+    assert _workspace(batch, q, keys, hq, hkv) == slots
 
 
 # (hq, hkv, longest query length): groups 2, 3, 4, 6, 8, 12, 16, 64; the last two
