@@ -322,16 +322,20 @@ struct SplitRule {
   int64_t slots;       // resident workgroups
   int64_t small_grid;  // grids up to here split whatever the range
   int64_t min_saved;   // else a chunk of at most half of it, or this many tiles saved
+  int64_t min_tiles;   // shorter ranges do not split
 };
 constexpr SplitRule kPrefillSplitRule = {kPrefillSlots, kPrefillSplitSmallGrid,
-                                         kPrefillSplitMinSaved};
+                                         kPrefillSplitMinSaved, 0};
 // Fused projection: one 256-row workgroup per CU, and a tile in the bias band costs
-// it about 3 us, so any underfilled grid splits when that saves four tiles.  Whole
-// calls without and with the split (one box, us, Hq 8 / Hkv 2, d 128, extent 1024,
-// bf16 r): 2 x 900..2100 tokens 86.0 -> 51.1, 1 x 1000 66.5 -> 32.8, 1 x 3000 117 -> 78,
-// 3 x 100..600 over 300..2000 keys bottom-right 102.5 -> 61.8, 3 x 2000 98.7 -> 93.0
-// (98.0 when 16 tiles had to be saved), 6 x 1200 (240 workgroups, no split) 76.
-constexpr SplitRule kProjSplitRule = {256, 256, 4};
+// it about 3 us, so any underfilled grid splits when that saves four tiles of a range of
+// eight.  Whole calls without and with the split (one box, us, Hq 8 / Hkv 2, d 128, extent
+// 1024, bf16 r): 2 x 900..2100 tokens 86.0 -> 51.1, 1 x 1000 66.5 -> 32.8, 1 x 3000 117 ->
+// 78, 3 x 100..600 over 300..2000 keys bottom-right 102.5 -> 61.8, window 255 6 x 300..400
+// (nine tiles) 41.5 -> 38.0, 3 x 2000 98.7 -> 93.0 (98.0 when 16 tiles had to be saved), 6 x
+// 1200 (240 workgroups, no split) 76.  Shorter ranges, split: 6 x 50..300 (five tiles) 24.0 ->
+// 25.9, 10 x 200 (four) 23.7 -> 29.7, 6 x 300..400 (six or seven) 28.4 -> 31.7, Hq 16 / Hkv 4
+// 28.4 -> 35.8.
+constexpr SplitRule kProjSplitRule = {256, 256, 4, 8};
 
 // bottom_right: the queries are the last of their sequence's keys.  The estimate
 // takes the longest cache for every sequence and, without a window, every key for
@@ -358,6 +362,7 @@ inline PrefillSplit prefill_split_for(int64_t batch, int64_t n_heads, int64_t ma
     // a short window leaves too few tiles to repay the merge pass (1 x 58..126
     // queries, window 127, five tiles: 14.3 us split)
     if (bottom_right && window_left >= 0 && tmax < 8) return s;
+    if (tmax < rule.min_tiles) return s;
     if (grid > rule.small_grid && tmax < kPrefillSplitWideMinTiles) return s;
     const int64_t balanced =
         ((total * batch * n_heads + rule.slots - 1) / rule.slots * kPrefillChunkPct + 99) / 100;

@@ -50,18 +50,35 @@ def test_rproj_split(cuda, lens_q, past, causal, window, bottom_right, head_dim,
         assert torch.equal(full[0], out) and torch.equal(full[1], lse)
 
 
-def test_rproj_workspace_on_the_host():
-    lib = _abi.lib()
+def _host_call(**kw):
     a = _abi.make_args(q=1 << 20, k=1 << 20, v=1 << 20, out=1 << 20, cu_seqlens_q=1 << 20,
                        cu_seqlens_k=1 << 20, q_stride_t=1024, q_stride_h=128, k_stride_t=256,
                        k_stride_h=128, v_stride_t=256, v_stride_h=128, out_stride_t=1024,
-                       out_stride_h=128, total_q=1000, total_k=1000, batch=1, n_heads=8,
-                       kv_heads=2, head_dim=128, rel_extent=128, rel_width=128,
-                       max_seqlen_q=1000, max_seqlen_k=1000, causal=1,
-                       qkv_dtype=_abi.IFA4_BF16, rel_dtype=_abi.IFA4_FP32)
+                       out_stride_h=128, n_heads=8, kv_heads=2, head_dim=128, rel_extent=128,
+                       rel_width=128, causal=1, qkv_dtype=_abi.IFA4_BF16,
+                       rel_dtype=_abi.IFA4_FP32, **kw)
     pr = _abi.Ifa4RelProj()
     pr.struct_size, pr.d_rel = ctypes.sizeof(_abi.Ifa4RelProj), 16
     pr.r, pr.wt, pr.r_stride_t, pr.r_stride_h = 1 << 20, 1 << 20, 128, 16
+    return a, pr
+
+
+# ranges of eight tiles on split; shorter ones were measured slower split
+@pytest.mark.parametrize("batch,q,keys,window,splits", [
+    (1, 512, 512, -1, True), (1, 448, 448, -1, False), (10, 200, 200, -1, False),
+    (6, 400, 400, -1, False), (2, 60, 500, -1, True), (2, 60, 400, -1, False),
+    (6, 400, 1900, 255, True), (6, 60, 1500, 255, False)])
+def test_rproj_splits_long_ranges(batch, q, keys, window, splits):
+    a, pr = _host_call(total_q=batch * q, total_k=batch * keys, batch=batch, max_seqlen_q=q,
+                       max_seqlen_k=keys, window_left=window,
+                       flags=_abi.IFA4_FLAG_BOTTOM_RIGHT if keys > q else 0)
+    n = _abi.lib().ifa4_prefill_rproj_workspace_bytes(ctypes.byref(a), ctypes.byref(pr))
+    assert (n > 0) == splits
+
+
+def test_rproj_workspace_on_the_host():
+    lib = _abi.lib()
+    a, pr = _host_call(total_q=1000, total_k=1000, batch=1, max_seqlen_q=1000, max_seqlen_k=1000)
     n = lib.ifa4_prefill_rproj_workspace_bytes(ctypes.byref(a), ctypes.byref(pr))
     assert n > 0
     for ws, size in ((None, 0), (1 << 20, n - 1), ((1 << 20) + 16, n)):
