@@ -193,6 +193,14 @@ ifa4::PrefillParams make_prefill_params(const ifa4_args* a) {
   return p;
 }
 
+// The call's bias is a shared table that the kernel stages in LDS.
+bool shared_table(const ifa4_args* a) {
+  ifa4::PrefillParams p{};
+  p.rel_st = a->rel_stride_t;
+  p.rel_extent = a->rel_extent;
+  return ifa4::prefill_tab(p);
+}
+
 // Query heads of a kv head whose rows share the query tiles: the whole group
 // when that takes fewer tiles (prefill_can_pack), the call gains by it (prefill_packs;
 // IFA4_FLAG_SPLIT_KV_2 packs without asking), and its q rows and bias rows stay
@@ -203,10 +211,7 @@ int prefill_pack(const ifa4_args* a) {
   const int64_t group = a->n_heads / a->kv_heads;
   const int bq = ifa4::prefill_block_q();
   if (!ifa4::prefill_can_pack(group, a->max_seqlen_q, bq)) return 1;
-  ifa4::PrefillParams p{};
-  p.rel_st = a->rel_stride_t;
-  p.rel_extent = a->rel_extent;
-  const bool table = ifa4::prefill_tab(p);
+  const bool table = shared_table(a);
   if ((a->flags & IFA4_FLAG_SPLIT_KV_2) == 0) {
     int64_t key_tiles, total;
     ifa4::prefill_tile_work(
@@ -235,7 +240,7 @@ ifa4::PrefillSplit prefill_split(const ifa4_args* a, int pack, bool proj = false
                                  (a->flags & IFA4_FLAG_NO_PRUNE) != 0,
                                  (proj ? ifa4::prefill_proj_block_q() : ifa4::prefill_block_q()) / pack,
                                  ifa4::prefill_block_k(),
-                                 (a->flags & IFA4_FLAG_SPLIT_KV_2) ? 2 : 0,
+                                 (a->flags & IFA4_FLAG_SPLIT_KV_2) ? 2 : 0, shared_table(a),
                                  proj ? ifa4::kProjSplitRule : ifa4::kPrefillSplitRule);
 }
 

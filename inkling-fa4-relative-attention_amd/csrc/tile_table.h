@@ -337,36 +337,63 @@ constexpr SplitRule kPrefillSplitRule = {kPrefillSlots, kPrefillSplitSmallGrid,
 // 28.4 -> 35.8.
 constexpr SplitRule kProjSplitRule = {256, 256, 4, 8};
 
+// Tiles of the longest range from which a windowed bottom-right call splits: the merge
+// pass costs about as much as four tiles of a per-token bias (2 us each) or six of a shared
+// table, and the more the more workgroups there are.  Split against not, by workgroups
+// without the split and tiles (one box, us, bf16 bias; t: shared table):
+//     4..12   4 tiles 12.3 / 11.6   5 13.5 / 15.0   7 13.4 / 17.3   t 5 12.7 / 12.1   t 6 11.9 / 12.7
+//    16..24   4 14.0 / 12.2         5 14.7 / 15.0   7 15.0 / 17.8   t 6 13.9 / 12.9   t 7 14.6 / 15.0
+//    32..48   4 14.6 / 12.1         5 14.7 / 14.2   6 14.7 / 15.9   t 6 12.2 / 12.5   t 8 12.6 / 15.0
+//    64..128  4 18.2 / 12.8         7 22.2 / 19.1   9 24.9 / 23.4   t 9 24.3 / 18.0   t 11 26.0 / 20.6
+//   144..288                                                       t 18 37.7 / 29.5  t 19 32.5 / 31.0
+inline int64_t window_split_tiles(int64_t grid, bool table) {
+  if (table) return grid < 16 ? 6 : grid < 32 ? 7 : grid < 64 ? 8 : grid <= 128 ? 12 : 32;
+  return grid < 32 ? 5 : grid < 64 ? 6 : 10;
+}
+// Shortest chunk of such a call from 64 workgroups on (chunks of two tiles against four:
+// window 511 8 x 128 queries over 1.5K keys 25.8 -> 23.6, window 700 4 x 256 with a
+// shared table 28.0 -> 22.4, window 1023 1 x 1000 over 200 keys 24.7 -> 26.8).
+constexpr int64_t kWindowMinChunk = 4;
+
 // bottom_right: the queries are the last of their sequence's keys.  The estimate
 // takes the longest cache for every sequence and, without a window, every key for
 // every query (the causal mask takes max_q keys at most).  With a window the
 // ranges are short wherever the queries sit: counting them so (instead of the
 // whole cache, us on one box): 3 x 300..500 queries, window 511, over 100..4000
 // keys 38.3 -> 26.3, 1 x 1000 32.9 -> 24.7, 6 x 20..40 22.5 -> 15.3.
-// no_prune: masked tiles are visited too (debug).  forced_chunk > 0: split every query tile into chunks of
-// that many tiles.
+// no_prune: masked tiles are visited too (debug).  forced_chunk > 0: split every query
+// tile into chunks of that many tiles.  table: the bias is a shared table.
 inline PrefillSplit prefill_split_for(int64_t batch, int64_t n_heads, int64_t max_q,
                                       int64_t max_k, bool causal, int64_t window_left,
                                       bool bottom_right, bool no_prune, int32_t block_q,
-                                      int32_t block_k, int32_t forced_chunk,
+                                      int32_t block_k, int32_t forced_chunk, bool table,
                                       const SplitRule& rule = kPrefillSplitRule) {
   PrefillSplit s{0, 1, 1};
   if (batch <= 0 || max_q <= 0 || max_k <= 0) return s;
-  const PrefillMasks masks = plan_masks(causal, window_left, bottom_right, max_q, max_k);
+  PrefillMasks masks = plan_masks(causal, window_left, bottom_right, max_q, max_k);
   int64_t tmax = 0, total = 0;
   prefill_tile_work(max_q, max_k, masks, block_q, block_k, &tmax, &total);
   int64_t chunk = forced_chunk;
   if (chunk <= 0) {
     const int64_t grid = (max_q + block_q - 1) / block_q * n_heads * batch;
     if (grid >= rule.slots || grid > kPrefillSplitMaxGrid) return s;
-    // a short window leaves too few tiles to repay the merge pass (1 x 58..126
-    // queries, window 127, five tiles: 14.3 us split)
-    if (bottom_right && window_left >= 0 && tmax < 8) return s;
     if (tmax < rule.min_tiles) return s;
+    bool windowed = bottom_right && window_left >= 0 && rule.min_tiles == 0;
+    if (windowed && tmax < window_split_tiles(grid, table)) return s;
     if (grid > rule.small_grid && tmax < kPrefillSplitWideMinTiles) return s;
+    if (windowed && 3 * (block_q + window_left) > 2 * max_k) {
+      // The window covers most of the cache: planned over all of it, in longer chunks
+      // (ranges of the window against it: window 1500, 2 x 2000 queries over 200 keys, Hq =
+      // Hkv = 4 40.0 -> 35.8; window 1023, 3 x 1000 over 200 43.7 -> 40.0, 30 x 128 over 1.5K,
+      // 4 heads 49.7 -> 45.1).
+      windowed = false;
+      masks = PrefillMasks{false, -1, 0};
+      prefill_tile_work(max_q, max_k, masks, block_q, block_k, &tmax, &total);
+    }
     const int64_t balanced =
         ((total * batch * n_heads + rule.slots - 1) / rule.slots * kPrefillChunkPct + 99) / 100;
-    chunk = balanced > kPrefillMinChunk ? balanced : kPrefillMinChunk;
+    const int64_t least = windowed && grid >= 64 ? kWindowMinChunk : kPrefillMinChunk;
+    chunk = balanced > least ? balanced : least;
     if (IFA4_PREFILL_CHUNK_FIT && chunk < tmax) {
       // Chunks of the balanced share can number a little more than the slots
       // (each query tile's last chunk is short): the few left over then run as

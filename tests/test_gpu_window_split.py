@@ -49,3 +49,35 @@ def test_windowed_chunks_cover_every_alignment(cuda, lens_q, past, window):
                              torch.bfloat16, seed=window, window_left=window, rel_table=False,
                              rel_extent=200, rel_dtype=torch.bfloat16, scale=0.1)
     _check(case, cuda)
+
+
+def _splits(batch, q, keys, hq, hkv, window, table):
+    a = _abi.make_args(q=1 << 20, k=1 << 20, v=1 << 20, out=1 << 20, cu_seqlens_q=1 << 20,
+                       cu_seqlens_k=1 << 20, rel=1 << 20, q_stride_t=hq * 128, q_stride_h=128,
+                       k_stride_t=hkv * 128, k_stride_h=128, v_stride_t=hkv * 128,
+                       v_stride_h=128, out_stride_t=hq * 128, out_stride_h=128,
+                       rel_stride_t=0 if table else hq * 512, rel_stride_h=512,
+                       total_q=batch * q, total_k=batch * keys, batch=batch, n_heads=hq,
+                       kv_heads=hkv, head_dim=128, rel_extent=512, rel_width=512,
+                       max_seqlen_q=q, max_seqlen_k=keys, causal=1, window_left=window,
+                       flags=_abi.IFA4_FLAG_BOTTOM_RIGHT, qkv_dtype=_abi.IFA4_BF16,
+                       rel_dtype=_abi.IFA4_BF16)
+    return _abi.lib().ifa4_prefill_workspace_bytes(a) > 0
+
+
+# short windows split where few workgroups make the merge pass cheap; (workgroups, tiles)
+@pytest.mark.parametrize("batch,q,keys,hq,hkv,window,table,splits", [
+    (1, 128, 4128, 8, 2, 255, False, True),     # 8, 7: 17.2 us without the split, 13.3 with it
+    (1, 128, 4128, 8, 2, 127, False, True),     # 8, 5
+    (1, 128, 4128, 8, 2, 63, False, False),     # 8, 4
+    (1, 128, 4128, 8, 2, 127, True, False),     # 8, 5, shared table
+    (1, 128, 4128, 8, 2, 255, True, True),      # 8, 7
+    (2, 500, 4500, 4, 4, 255, False, True),     # 32, 7
+    (2, 500, 4500, 8, 2, 255, False, False),    # 64, 7: 18.7 us without the split, 22.9 with it
+    (1, 1000, 5000, 8, 2, 511, False, True),    # 64, 11
+    (1, 1000, 5000, 8, 2, 511, True, False),    # 64, 11, shared table
+    (20, 128, 6128, 8, 2, 1023, True, False),   # 160, 18, shared table
+    (20, 128, 6128, 8, 2, 1023, False, True),   # 160, 18
+])
+def test_short_windows_split_small_grids(batch, q, keys, hq, hkv, window, table, splits):
+    assert _splits(batch, q, keys, hq, hkv, window, table) == splits
