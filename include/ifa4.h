@@ -141,7 +141,8 @@ typedef struct ifa4_rel_proj {
 
 /* Tile shape chosen for a call (the gfx950 tile table). */
 typedef struct ifa4_tile {
-  int32_t block_q;        /* query rows per workgroup */
+  int32_t block_q;        /* query rows per workgroup (prefill calls of a few queries per
+                             sequence may take rows of several query heads of a kv head) */
   int32_t block_k;        /* keys per KV tile */
   int32_t waves;          /* wavefronts per workgroup */
   int32_t stages;         /* LDS buffers for K/V */

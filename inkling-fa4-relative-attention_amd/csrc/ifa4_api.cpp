@@ -511,8 +511,11 @@ int32_t ifa4_prefill_tile(const ifa4_args* args, ifa4_tile* tile) {
       tile->block_k = e.block_k;
       tile->waves = e.waves;
       tile->stages = e.stages;
-      // split KV (ifa4_prefill_fwd_ws): keys per chunk, 0 when the call does not split
-      const ifa4::PrefillSplit sp = prefill_split(args, 1);
+      // split KV (ifa4_prefill_fwd_ws): keys per chunk, 0 when the call does not split.
+      // The arguments may be a shape alone, without heads or tensors to check.
+      const bool heads = args->n_heads > 0 && args->kv_heads > 0 &&
+                         args->n_heads % args->kv_heads == 0;
+      const ifa4::PrefillSplit sp = prefill_split(args, heads ? prefill_pack(args) : 1);
       tile->kv_chunk = sp.chunk_tiles * e.block_k;
       return IFA4_OK;
     }

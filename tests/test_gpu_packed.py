@@ -8,6 +8,8 @@ always under the test flag of two-tile chunks, so every case runs both ways.
 Everything is compared with the fp32 oracle (16-bit rounding of P and of the output:
 2e-2; fp32 LSE: 1e-3), and pruned with unpruned launches bit for bit.
 """
+import ctypes
+
 import pytest
 import torch
 
@@ -42,8 +44,8 @@ def _check(case, dev, bottom_right=True):
     torch.testing.assert_close(runs[1][0].float(), runs[0][0].float(), atol=2e-2, rtol=2e-2)
 
 
-def _workspace(batch, q, keys, hq, hkv, d=128, **kw):
-    """Workspace of a bottom-right call, and the chunk slots it holds."""
+def _host_args(batch, q, keys, hq, hkv, d=128, **kw):
+    """A bottom-right call with a per-token bias, for the host-side queries."""
     fields = dict(q=1 << 20, k=1 << 20, v=1 << 20, out=1 << 20, cu_seqlens_q=1 << 20,
                   cu_seqlens_k=1 << 20, rel=1 << 20, q_stride_t=hq * d, q_stride_h=d,
                   k_stride_t=hkv * d, k_stride_h=d, v_stride_t=hkv * d, v_stride_h=d,
@@ -53,8 +55,7 @@ def _workspace(batch, q, keys, hq, hkv, d=128, **kw):
                   causal=1, flags=_abi.IFA4_FLAG_BOTTOM_RIGHT, qkv_dtype=_abi.IFA4_BF16,
                   rel_dtype=_abi.IFA4_BF16)
     fields.update(kw)
-    n = _abi.lib().ifa4_prefill_workspace_bytes(_abi.make_args(**fields))
-    return n // (hq * batch * q * (d + 1) * 4)
+    return _abi.make_args(**fields)
 
 
 # chunk slots of the plan without packed rows (per head) and with them, and which of
@@ -69,7 +70,13 @@ def _workspace(batch, q, keys, hq, hkv, d=128, **kw):
     (16, 32, 8032, 8, 2, 16),    # packed: 32 workgroups in chunks of eight (unpacked: four slots)
 ])
 def test_packed_where_it_pays(batch, q, keys, hq, hkv, slots):
-    assert _workspace(batch, q, keys, hq, hkv) == slots
+    a = _host_args(batch, q, keys, hq, hkv)
+    n = _abi.lib().ifa4_prefill_workspace_bytes(a)
+    assert n // (hq * batch * q * (128 + 1) * 4) == slots
+    # the tile query reports the chunks that run
+    tile = _abi.Ifa4Tile()
+    assert _abi.lib().ifa4_prefill_tile(a, ctypes.byref(tile)) == _abi.IFA4_OK
+    assert (-(-keys // tile.kv_chunk) if tile.kv_chunk else 0) == slots
 
 
 # (hq, hkv, longest query length): groups 2, 3, 4, 6, 8, 12, 16, 64; the last two
