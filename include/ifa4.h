@@ -220,12 +220,13 @@ int32_t ifa4_prefill_count_tiles(const ifa4_args* args, const int32_t* host_cu_s
  * when adjacent kv heads stream in pairs, 1536 paged, else 2048; fewer for
  * small calls) over all (sequence, kv head) caches laid end to end in 32-key
  * steps, each wave an equal range of work (a step whose keys carry bias
- * counts 7/4 of a plain one; ifa4_decode_tile reports the keys per wave of a
- * contiguous 16-bit cache); it writes one (o, lse) partial per (cache, wave)
+ * counts 7/4 of a plain one); it writes one (o, lse) partial per (cache, wave)
  * it touches into the workspace.  Pass 2 merges each cache's partials by log-sum-exp and
- * writes out/lse.  Calls of short caches or windows (up to 20 steps of 32 keys, more
- * when the caches are many) take one launch instead, a workgroup per cache, and leave
- * the workspace untouched.  The workspace (ifa4_decode_workspace_bytes, 256-byte
+ * writes out/lse.  Calls of short caches or windows (up to 20 steps of 32 keys, 32 from
+ * 128 (sequence, kv head) caches on; half of that for GQA groups above 8) take one launch
+ * instead, a workgroup of 8 (4) waves per cache, and leave the workspace untouched.
+ * ifa4_decode_tile reports the waves per workgroup and the most keys one wave
+ * streams for a contiguous 16-bit cache.  The workspace (ifa4_decode_workspace_bytes, 256-byte
  * aligned, contents on entry irrelevant) is scratch for one call; calls that
  * share a workspace must not overlap.  Replaces
  * inkling_fa4_rel_attention_decode_triton

@@ -354,6 +354,20 @@ int32_t decode_waves(const ifa4_args* a, bool fp8 = false, bool paged = false) {
                                 v.pair);
 }
 
+// One launch for the whole call: waves of its workgroups (ifa4::decode_whole), or 0 for
+// the stream and combine passes; *steps the steps of the longest cache.
+int32_t decode_whole_waves(const ifa4_args* a, const DecodeView& v, int64_t* steps) {
+  // visible keys, and one step more for the partial one a window may begin with
+  int64_t keys = key0_only(a) ? (a->max_seqlen_k > 0 ? 1 : 0) : a->max_seqlen_k;
+  if ((a->flags & IFA4_FLAG_BOTTOM_RIGHT) != 0 && a->window_left >= 0 &&
+      keys > (int64_t)a->window_left + ifa4::kDecodeStep)
+    keys = (int64_t)a->window_left + ifa4::kDecodeStep;
+  *steps = (keys + ifa4::kDecodeStep - 1) / ifa4::kDecodeStep;
+  return ifa4::decode_whole((int64_t)a->batch * v.kv_heads, v.group, *steps)
+             ? (int32_t)ifa4::decode_whole_waves(v.group)
+             : 0;
+}
+
 // Decode workspace: partial (o, lse) slots, one per (segment, wave) pair that
 // can exist (batch * kv_heads + waves, in the kernels' view of the kv heads),
 // then the per-segment wave ranges.
@@ -445,13 +459,8 @@ int32_t run_decode(const ifa4_args* args, const ifa4_paged_kv* kv, const ifa4_kv
   p.window_left = args->window_left < (1 << 30) ? args->window_left : (1 << 30);
   p.rel_dtype = args->rel_dtype;
   p.n_waves = decode_waves(args, qt != nullptr, kv != nullptr);
-  // steps of the longest cache: its visible keys, and one more for the partial
-  // step a window may begin with
-  int64_t keys = key0_only(args) ? (args->max_seqlen_k > 0 ? 1 : 0) : args->max_seqlen_k;
-  if (p.bottom_right && p.window_left >= 0 && keys > p.window_left + ifa4::kDecodeStep)
-    keys = p.window_left + ifa4::kDecodeStep;
-  p.whole = ifa4::decode_whole((int64_t)args->batch * view.kv_heads, view.group,
-                               (keys + ifa4::kDecodeStep - 1) / ifa4::kDecodeStep);
+  int64_t steps;
+  p.whole = decode_whole_waves(args, view, &steps) > 0 ? 1 : 0;
   p.kv_fp8 = qt != nullptr ? 1 : 0;
   p.scale_log2 = args->softmax_scale * (qt != nullptr ? qt->k_scale : 1.f) * kLog2eHost;
   p.v_scale = qt != nullptr ? qt->v_scale : 1.f;
@@ -615,12 +624,21 @@ int32_t ifa4_decode_tile(const ifa4_args* args, ifa4_tile* tile) {
   if (tile == nullptr) return IFA4_EINVAL;
   const int32_t st = check_decode(args);
   if (st != IFA4_OK) return st;
-  // One wave per workgroup, 32-key steps, two register stages; kv_chunk = the
-  // most keys one persistent wave streams (ceil(steps / waves) steps).
+  // 32-key steps, two register stages; kv_chunk = the most keys one wave streams:
+  // its share of the longest cache where one launch takes the call (a workgroup of
+  // `waves` waves per cache), else ceil(steps / waves) steps of the persistent waves, one
+  // a workgroup.
   tile->block_q = 1;
   tile->block_k = ifa4::kDecodeStep;
-  tile->waves = 1;
   tile->stages = 2;
+  int64_t longest;
+  if (const int32_t nw = args->batch > 0 ? decode_whole_waves(args, decode_view(args, false), &longest)
+                                         : 0) {
+    tile->waves = nw;
+    tile->kv_chunk = (int32_t)((longest + nw - 1) / nw * ifa4::kDecodeStep);
+    return IFA4_OK;
+  }
+  tile->waves = 1;
   const int64_t steps = ifa4::decode_max_steps(args->batch, args->kv_heads, args->max_seqlen_k,
                                                key0_only(args));
   const int32_t w = decode_waves(args);

@@ -132,8 +132,10 @@ inline bool decode_pairs(bool fp8, int64_t head_dim, int64_t kv_heads, int64_t g
 //   200..6000 paged keys 24 sequences 15.9 -> 14.0, 64 20.8 -> 15.0; window 1023
 //   (33 steps) 16.9 -> 21.1.
 // With 4 waves a segment everything but 64 x 256 is slower (64 x 512 13.4, windows 18.5).
+// Groups above 8 take half the waves: their Q rows and tiles fill the LDS.
+constexpr int64_t decode_whole_waves(int64_t group) { return group > 8 ? 4 : 8; }
 inline bool decode_whole(int64_t segments, int64_t group, int64_t max_steps) {
-  const int64_t waves = group > 8 ? 4 : 8;
+  const int64_t waves = decode_whole_waves(group);
   if (2 * max_steps <= 5 * waves) return true;
   return max_steps <= 4 * waves && segments >= 128;
 }

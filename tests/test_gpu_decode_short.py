@@ -7,10 +7,12 @@ or with two queries.  Against the fp32 oracle (16-bit rounding of P and of the o
 2e-2; LSE 1e-3) on every cache format; a longer cache in max_seqlen_k sends the same
 sequences through the two-pass kernels, which must agree (LSE 1e-4).
 """
+import ctypes
+
 import pytest
 import torch
 
-from inkling_fa4 import (inkling_fa4_rel_attention_decode, inkling_fa4_rel_attention_decode_paged,
+from inkling_fa4 import (_abi, inkling_fa4_rel_attention_decode, inkling_fa4_rel_attention_decode_paged,
                          testing)
 from oracle import ref_rel_attn_with_lse
 
@@ -104,3 +106,24 @@ def test_short_rows_without_exactly_one_query(cuda):
         softmax_scale=c.scale, return_lse=True)
     assert bool((out[:2] == 0).all()) and bool((lse[:, :2] == float("-inf")).all())
     assert torch.equal(out[2], ref[0][2]) and torch.equal(lse[:, 2], ref[1][:, 2])
+
+
+# (waves per workgroup, keys per wave) that the tile query reports: the one-launch form on
+# both sides of its rule, and the persistent waves
+@pytest.mark.parametrize("batch,keys,hq,hkv,window,waves,chunk", [
+    (1, 512, 8, 2, -1, 8, 64), (1, 640, 8, 2, -1, 8, 96), (1, 641, 8, 2, -1, 1, 64),
+    (64, 1024, 8, 2, -1, 8, 128), (64, 1025, 8, 2, -1, 1, 160), (63, 1024, 8, 2, -1, 1, 160),
+    (1, 320, 16, 1, -1, 4, 96), (1, 321, 16, 1, -1, 1, 64), (24, 16384, 8, 2, 511, 8, 96),
+    (24, 16384, 8, 2, 1023, 1, 896), (4, 0, 8, 2, -1, 8, 0)])
+def test_decode_tile_reports_what_runs(batch, keys, hq, hkv, window, waves, chunk):
+    a = _abi.make_args(q=1 << 20, k=1 << 20, v=1 << 20, out=1 << 20, cu_seqlens_q=1 << 20,
+                       cu_seqlens_k=1 << 20, q_stride_t=hq * 128, q_stride_h=128,
+                       k_stride_t=hkv * 128, k_stride_h=128, v_stride_t=hkv * 128,
+                       v_stride_h=128, out_stride_t=hq * 128, out_stride_h=128, total_q=batch,
+                       total_k=batch * keys, batch=batch, n_heads=hq, kv_heads=hkv, head_dim=128,
+                       max_seqlen_q=1, max_seqlen_k=keys, causal=1, window_left=window,
+                       flags=_abi.IFA4_FLAG_BOTTOM_RIGHT, qkv_dtype=_abi.IFA4_BF16,
+                       rel_dtype=_abi.IFA4_BF16)
+    tile = _abi.Ifa4Tile()
+    assert _abi.lib().ifa4_decode_tile(a, ctypes.byref(tile)) == _abi.IFA4_OK
+    assert (tile.block_k, tile.waves, tile.kv_chunk) == (32, waves, chunk)
