@@ -203,9 +203,11 @@ int32_t ifa4_prefill_rproj_fwd_ws(const ifa4_args* args, const ifa4_rel_proj* pr
 int32_t ifa4_prefill_tile(const ifa4_args* args, ifa4_tile* tile);
 
 /*
- * Host-side count of the KV tiles the prefill kernel visits, using the same
+ * Host-side count of the KV tiles ifa4_prefill_fwd visits, using the same
  * pruning rule as the device code, from host copies of cu_seqlens.  total =
- * tiles an unpruned kernel would visit.  For reports and tests.
+ * tiles an unpruned kernel would visit.  A call that packs query heads visits a tile
+ * once for all of them; without kv_heads and max_seqlen_q/k, one head per tile is
+ * counted.  For reports and tests.
  */
 int32_t ifa4_prefill_count_tiles(const ifa4_args* args, const int32_t* host_cu_seqlens_q,
                                  const int32_t* host_cu_seqlens_k, int64_t* visited,

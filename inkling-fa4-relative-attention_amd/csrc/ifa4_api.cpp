@@ -262,6 +262,14 @@ PrefillWorkspace prefill_workspace(const ifa4_args* a, bool proj = false) {
   return w;
 }
 
+// Packed rows of the call without a workspace: those of ifa4_prefill_fwd_ws where that
+// needs none, so that both run the same; one head per tile where it would split (a
+// packed range in one piece keeps all its waves busy for as long: no gain).
+int unsplit_pack(const ifa4_args* a) {
+  const PrefillWorkspace w = prefill_workspace(a);
+  return w.total() == 0 ? w.pack : 1;
+}
+
 // The split of a call in its workspace; false when that is missing or too small.
 bool set_split(ifa4::PrefillParams& p, const PrefillWorkspace& w, void* workspace,
                size_t workspace_bytes) {
@@ -536,7 +544,8 @@ int32_t ifa4_prefill_fwd(const ifa4_args* args, void* stream) {
   const int32_t st = check_args(args);
   if (st != IFA4_OK) return st;
   if (args->batch == 0 || args->max_seqlen_q == 0) return IFA4_OK;
-  const ifa4::PrefillParams p = make_prefill_params(args);
+  ifa4::PrefillParams p = make_prefill_params(args);
+  set_tiles(p, args, ifa4::prefill_block_q(), unsplit_pack(args));
   const hipError_t e = ifa4::launch_prefill(p, args->head_dim, args->qkv_dtype,
                                             static_cast<hipStream_t>(stream));
   return e == hipSuccess ? IFA4_OK : IFA4_ELAUNCH;
@@ -584,8 +593,12 @@ int32_t ifa4_prefill_count_tiles(const ifa4_args* args, const int32_t* cu_q, con
       total == nullptr)
     return IFA4_EINVAL;
   if (args->batch < 0 || args->n_heads < 1) return IFA4_EINVAL;
-  const int bq = ifa4::prefill_block_q();
+  // packed rows need the heads and lengths of the call; a shape without them has none
+  const int pack =
+      args->kv_heads > 0 && args->n_heads % args->kv_heads == 0 ? unsplit_pack(args) : 1;
+  const int bq = ifa4::prefill_block_q() / pack;  // queries per tile
   const int bk = ifa4::prefill_block_k();
+  const int heads = args->n_heads / pack;  // tiles side by side
   const bool no_prune = (args->flags & IFA4_FLAG_NO_PRUNE) != 0;
   const bool bottom_right = (args->flags & IFA4_FLAG_BOTTOM_RIGHT) != 0;
   int64_t vis = 0, tot = 0;
@@ -606,8 +619,8 @@ int32_t ifa4_prefill_count_tiles(const ifa4_args* args, const int32_t* cu_q, con
       }
       const int kt_beg = kbeg / bk;
       const int kt_end = kend > kbeg ? (kend + bk - 1) / bk : kt_beg;
-      vis += (int64_t)(kt_end - kt_beg) * args->n_heads;
-      tot += (int64_t)((lk + bk - 1) / bk) * args->n_heads;
+      vis += (int64_t)(kt_end - kt_beg) * heads;
+      tot += (int64_t)((lk + bk - 1) / bk) * heads;
     }
   }
   *visited = vis;

@@ -79,6 +79,48 @@ def test_packed_where_it_pays(batch, q, keys, hq, hkv, slots):
     assert (-(-keys // tile.kv_chunk) if tile.kv_chunk else 0) == slots
 
 
+def test_count_of_packed_tiles():
+    # 200 x 8 queries over 308 keys: more workgroups than fit at once, packed, not split
+    a = _host_args(200, 8, 308, 8, 2)
+    assert _abi.lib().ifa4_prefill_workspace_bytes(a) == 0
+    cu_q = (ctypes.c_int32 * 201)(*range(0, 201 * 8, 8))
+    cu_k = (ctypes.c_int32 * 201)(*range(0, 201 * 308, 308))
+    vis, tot = ctypes.c_int64(), ctypes.c_int64()
+    assert _abi.lib().ifa4_prefill_count_tiles(a, cu_q, cu_k, ctypes.byref(vis),
+                                               ctypes.byref(tot)) == _abi.IFA4_OK
+    assert vis.value == tot.value == 200 * 2 * 5  # one tile per kv head, five KV tiles
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hq,hkv", [(8, 2), (6, 2)])
+def test_no_workspace_runs_the_same(cuda, hq, hkv):
+    # a call that needs no workspace: ifa4_prefill_fwd and ifa4_prefill_fwd_ws bit for bit
+    lens_q = [1 + i % 8 for i in range(200)]
+    lens_k = [n + (i * 37) % 300 for i, n in enumerate(lens_q)]
+    case = testing.make_case("no_ws", lens_q, lens_k, hq, hkv, 128, torch.bfloat16, seed=hq,
+                             rel_table=False, rel_extent=200, rel_dtype=torch.bfloat16, scale=0.1)
+    print(f"no workspace, {hq}/{hkv} heads", flush=True)
+    c = case.to(cuda)
+    out, lse = _run(c)
+    got, got_lse = torch.empty_like(out), torch.empty_like(lse)
+    a = _abi.make_args(
+        q=c.q.data_ptr(), k=c.k.data_ptr(), v=c.v.data_ptr(), rel=c.rel.data_ptr(),
+        out=got.data_ptr(), lse=got_lse.data_ptr(), cu_seqlens_q=c.cu_q.data_ptr(),
+        cu_seqlens_k=c.cu_k.data_ptr(), q_stride_t=c.q.stride(0), q_stride_h=c.q.stride(1),
+        k_stride_t=c.k.stride(0), k_stride_h=c.k.stride(1), v_stride_t=c.v.stride(0),
+        v_stride_h=c.v.stride(1), rel_stride_t=c.rel.stride(0), rel_stride_h=c.rel.stride(1),
+        out_stride_t=got.stride(0), out_stride_h=got.stride(1), lse_stride_h=got_lse.stride(0),
+        total_q=sum(lens_q), total_k=sum(lens_k), batch=200, n_heads=hq, kv_heads=hkv,
+        head_dim=128, rel_extent=200, rel_width=200, max_seqlen_q=c.max_q, max_seqlen_k=c.max_k,
+        causal=1, softmax_scale=c.scale, flags=_abi.IFA4_FLAG_BOTTOM_RIGHT,
+        qkv_dtype=_abi.IFA4_BF16, rel_dtype=_abi.IFA4_BF16)
+    assert _abi.lib().ifa4_prefill_workspace_bytes(a) == 0
+    stream = torch.cuda.current_stream().cuda_stream
+    assert _abi.lib().ifa4_prefill_fwd(a, stream) == _abi.IFA4_OK
+    torch.cuda.synchronize()
+    assert torch.equal(got, out) and torch.equal(got_lse, lse)
+
+
 # (hq, hkv, longest query length): groups 2, 3, 4, 6, 8, 12, 16, 64; the last two
 # lengths of each are the edge of the rule and just past it
 @pytest.mark.gpu
