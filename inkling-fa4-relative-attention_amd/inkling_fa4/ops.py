@@ -80,8 +80,12 @@ def _call(name, *args):
         op = _overloads[name] = getattr(_ops(), name).default
     if _is_grad_enabled():
         q, k, v, rel, w = args[:5]
-        if (q.requires_grad or k.requires_grad or v.requires_grad or rel.requires_grad
-                or w.requires_grad):
+        try:
+            off = (q.requires_grad or k.requires_grad or v.requires_grad or rel.requires_grad
+                   or w.requires_grad)
+        except AttributeError:  # not a tensor: the operator says so
+            off = False
+        if off:
             with torch.no_grad():
                 return op(*args)
     return op(*args)

@@ -27,3 +27,10 @@ def test_outputs_never_require_grad(cuda, grad, which):
         out = inkling_fa4_rel_attention_rproj(c.q, c.k, c.v, r, w.requires_grad_(which == 4),
                                               *c.args()[4:])
         assert not out.requires_grad
+
+
+@pytest.mark.parametrize("grad", [True, False])
+def test_other_objects_are_refused_by_the_operator(grad):
+    c = testing.make_case("none", [3], [3], 4, 2, 64, torch.bfloat16, seed=1)
+    with torch.set_grad_enabled(grad), pytest.raises(RuntimeError):
+        inkling_fa4_rel_attention(c.q, c.k, c.v, None, *c.args()[4:])
