@@ -1000,12 +1000,10 @@ decode_stream_kernel(DecodeParams p) {
     // writes that before the barrier), [head][D] fp32; a thread then owns a 16-byte
     // chunk of a head's row over all waves.
     constexpr int kHeads = G < 16 ? G : 16;
-    static_assert(kHeads * D * 4 <= (int)sizeof(k_tiles[0]) + (int)sizeof(v_tiles[0]),
-                  "a wave's partial fits its tiles");
-    constexpr bool kInK = kHeads * D * 4 <= (int)sizeof(k_tiles[0]);
+    static_assert(kHeads * D * 4 <= (int)sizeof(k_tiles[0]), "a wave's partial fits its K tile");
     __shared__ float part_m[kW][kHeads], part_l[kW][kHeads];
     const float l_tot = add_xor32(add_xor16(l_run));
-    float* const mine = reinterpret_cast<float*>(kInK ? k_lds : v_lds);
+    float* const mine = reinterpret_cast<float*>(k_lds);
     if (n < g_act) {
 #pragma unroll
       for (int db = 0; db < S::kDBlocks; ++db)
@@ -1029,8 +1027,8 @@ decode_stream_kernel(DecodeParams p) {
       for (int i = 0; i < kW; ++i) {
         const float a = fast_exp2(part_m[i][h] - mu);
         lt += a * part_l[i][h];
-        out += a * *reinterpret_cast<const f32x4_t*>(
-                       reinterpret_cast<const float*>(kInK ? k_tiles[i] : v_tiles[i]) + h * D + d);
+        out += a * *reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(k_tiles[i]) +
+                                                     h * D + d);
       }
       const float inv = lt > 0.f ? p.v_scale / lt : 0.f;
       const int head = cur[0].kvh * g_act + h;
