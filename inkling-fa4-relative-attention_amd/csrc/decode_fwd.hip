@@ -55,8 +55,9 @@
 // the launches; see the figures at decode_whole.
 //
 // Pass 2 (decode_combine_kernel): per (head, sequence) merge of the segment's
-// partials by log-sum-exp (16 part groups of a workgroup each merge online,
-// then meet in LDS); writes out (q dtype) and lse (natural log).
+// partials by log-sum-exp (a workgroup's part groups each merge online, those of a
+// wave meet by lane exchange, the eight waves in LDS); writes out (q dtype) and lse
+// (natural log).
 #include "ifa4_device.hpp"
 #include "ifa4_kernels.h"
 
@@ -916,7 +917,7 @@ decode_stream_kernel(DecodeParams p) {
       // segment (between two of its steps' starts), the segment's partials run
       // over this wave's slot too: an empty one (nothing seen) goes there.
       if (g0 >= cur[0].seg_u0) {
-  #pragma unroll
+#pragma unroll
         for (int db = 0; db < S::kDBlocks; ++db) o[db] = f32x4_t{};
         put_partial(cur[0].seg + w, 0.f, -INFINITY);
       }
@@ -1051,9 +1052,9 @@ constexpr int kWholeWaves = 8;  // waves of a one-launch workgroup
 // sequence bounds and the segment's wave range (independent loads), then the
 // parts themselves.  Thread (g, c) holds chunk c and merges parts g, g +
 // kGroups, ... online (running max, rescaled sums, four parts' loads in
-// flight); the kGroups results of a chunk meet in LDS.  With 8 waves that is
-// 16 groups per split at D = 128 (32 at D = 64), so a segment of up to 64
-// (128) parts per split merges in one round of loads.  The host takes more
+// flight); a wave's groups then meet by lane exchange and the eight waves in LDS.
+// With 8 waves that is 16 groups at D = 128 (32 at D = 64) times SPLIT, so a segment
+// of up to 64 (128) parts per split merges in one round of loads.  The host takes more
 // splits for segments of many parts (a few long caches spread over many
 // waves: one sequence of 128K keys over 1024 waves has ~512 parts per cache).
 // Every split merges the same parts in the same order, so the running max and

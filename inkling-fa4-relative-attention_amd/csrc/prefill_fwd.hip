@@ -301,7 +301,7 @@ __device__ __forceinline__ void prefill_work(const PrefillParams& p, const WorkI
   constexpr int kBiasLdsFloats = kPack ? kBiasPackFloats : 2 * kBiasPad + kBiasLdsMax;
   constexpr int kDBlocks = D / 32;
   constexpr int kKSteps = D / 16;
-  static_assert(!kPack || kNqb == 1, "packed rows: one row block per wave");
+  static_assert(!kPack || (kNqb == 1 && !kProj), "packed rows: one row block per wave");
 
   // Both stages in one array: a read of stage 1 is the stage-0 address plus a
   // constant, which folds into the instruction's offset (one address register
@@ -536,7 +536,7 @@ __device__ __forceinline__ void prefill_work(const PrefillParams& p, const WorkI
   constexpr bool kProjEarly = IFA4_PROJ_EARLY;
   auto proj_bias = [&](int kb, int blk, float* bias) {
     if (!(kProjEarly && blk == 0)) proj_fill(kb, blk);
-    const float* src = mp + col * kProjPitch + (qi[0] - imin) + 31 - 16 * half;
+    const float* src = mp + col * (kProjPitch + 1) + 31 - 16 * half;
 #pragma unroll
     for (int e = 0; e < 16; ++e) bias[e] = src[-e];
   };
@@ -1186,10 +1186,7 @@ __device__ __forceinline__ void prefill_work(const PrefillParams& p, const WorkI
   // operand, and the first tile's W^T rows.
   if constexpr (kProj) {
     float rv[8];
-    const uint32_t roff =
-        !kPack || row_ok[0]
-            ? (uint32_t)(qi[0] * (int)p.rel_st + hq[0] * (int)p.rel_sh + 8 * half) * Rel::kBytes
-            : kOutOfRange;
+    const uint32_t roff = (uint32_t)(qi[0] * (int)p.rel_st + 8 * half) * Rel::kBytes;
 #pragma unroll
     for (int c = 0; c < 8; ++c) rv[c] = Rel::load(rrel, roff + c * Rel::kBytes);
     split_bf16x8(rv, r_hi, r_lo);
@@ -1225,7 +1222,7 @@ __device__ __forceinline__ void prefill_work(const PrefillParams& p, const WorkI
     const int qi_e = q0 + ql_e;
     const int head_e = kPack ? head + r_e - ql_e * pack : head;
     const bool ok_e = qi_e < it.q_end;
-if (ok_e && it.part >= 0) {
+    if (ok_e && it.part >= 0) {
       // normalised O of the chunk (fp32) and its LSE in log2 units
       const int64_t prow = ((int64_t)it.part * p.n_heads + head_e) * p.total_q + qs + qi_e;
       float* pbase = p.part_o + prow * D;
