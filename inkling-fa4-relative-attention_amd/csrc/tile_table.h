@@ -272,8 +272,9 @@ inline bool prefill_can_pack(int64_t group, int64_t max_q, int64_t block_q) {
 //     64 x 17..96 over Hq 16 / Hkv 2 21.2 -> 19.7;
 //   - ranges of 16 tiles on, where half of the 32-row waves go (12 x 2..5 queries over
 //     1K..8K keys 42.4 -> 22.9, 4 x 16 over 14K 31.6 -> 22.6), or the ranges together
-//     are 6000 tiles of up to 32 queries, or of any if they are 64 on (16 x 32 over 8K
-//     64.3 -> 46.1, 64 x 24 over 2K 57.3 -> 43.1, 4 x 64 over 14K 41.6 -> 34.8);
+//     are 6000 tiles of up to 32 queries, or of any if they are 64 on, or 3000 if 128 on (16
+//     x 32 over 8K 64.3 -> 46.1, 64 x 24 over 2K 57.3 -> 43.1, 4 x 64 over 14K 41.6 -> 34.8, 3 x
+//     20..40 over 3K..9K 26.7 -> 22.3, x 50..96 30.9 -> 28.9);
 //   - where three quarters of the waves go and the bias is per token: 64 x 2 over 500
 //     keys 17.5 -> 14.3 (shared table, whose tiles are cheap, x 8 14.3 -> 15.9).
 // Without one of these it measured (packed against not): 64 x 32 over 500 keys 20.4 ->
@@ -284,8 +285,9 @@ inline bool prefill_packs(int64_t grid, int64_t key_tiles, int64_t group, int64_
                           bool table) {
   const int64_t waves = group * ((max_q + 31) / 32), packed = (max_q * group + 31) / 32;
   if (grid > kPrefillSlots) return true;
+  const int64_t enough = key_tiles >= 128 ? 3000 : 6000;
   if (key_tiles >= 16 &&
-      (2 * packed <= waves || (grid * key_tiles >= 6000 && (max_q <= 32 || key_tiles >= 64))))
+      (2 * packed <= waves || (grid * key_tiles >= enough && (max_q <= 32 || key_tiles >= 64))))
     return true;
   return !table && 4 * packed <= waves && grid * key_tiles >= 512;
 }

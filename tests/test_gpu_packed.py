@@ -67,6 +67,7 @@ def _host_args(batch, q, keys, hq, hkv, d=128, **kw):
     (4, 64, 4064, 8, 2, 16),     # 32 workgroups in chunks of four tiles (packed: two, 32 slots)
     (12, 5, 8005, 8, 2, 21),     # packed: 24 workgroups in chunks of six (unpacked: 25, six)
     (64, 24, 2024, 8, 2, 4),     # packed: 128 in chunks of eight (unpacked: not split)
+    (3, 40, 9040, 8, 2, 36),     # packed: 12 workgroups in chunks of four (unpacked: 21 of seven)
     (16, 32, 8032, 8, 2, 16),    # packed: 32 workgroups in chunks of eight (unpacked: four slots)
 ])
 def test_packed_where_it_pays(batch, q, keys, hq, hkv, slots):
