@@ -1437,8 +1437,8 @@ hipError_t launch_prefill_t(const PrefillParams& p_in, hipStream_t stream) {
   // workgroups with work, from the rows: a last tile half full per sequence and head
   const int64_t live = ((int64_t)p.total_q / p.q_step + p.batch / 2) * p.tile_heads;
   const int64_t slots = 256 * (Sh::kWavesPerSimd * 4 / Sh::kWaves);  // resident workgroups
-  p.order = workgroup_order(p.tile_heads, p.tile_group, p.batch, p.ragged, p.n_qtiles, p.n_chunks,
-                            live, slots, kProj);
+  p.order = workgroup_order(OrderShape{p.tile_heads, p.tile_group, p.batch, p.ragged, p.n_qtiles,
+                                       p.n_chunks, live, slots, p.window_left >= 0, kProj});
   const int64_t blocks = order_blocks(p.order) * p.n_qtiles * p.n_chunks;
   if (blocks <= 0) return hipSuccess;
   hipLaunchKernelGGL((prefill_fwd_kernel<Sh, D, Tag, Rel, kProj, kTab, kPack>), dim3((unsigned)blocks),

@@ -18,9 +18,9 @@ SRC = r"""
 using namespace ifa4;
 // 0 when the workgroups of the call take every place exactly once
 extern "C" int check(int heads, int group, int batch, int ragged, int chunks, long live,
-                     long slots, int proj, int qtiles, int* form) {
-  const WorkgroupOrder o = workgroup_order(heads, group, batch, ragged, qtiles, chunks, live,
-                                           slots, proj);
+                     long slots, int windowed, int proj, int qtiles, int* form) {
+  const WorkgroupOrder o = workgroup_order(OrderShape{
+      heads, group, batch, ragged, qtiles, chunks, live, slots, windowed != 0, proj != 0});
   form[0] = o.lanes;
   form[1] = o.pair_heads;
   form[2] = o.lanes && !o.pair_heads ? 1 << o.spread_log : 0;
@@ -53,12 +53,12 @@ def lib(tmp_path_factory):
     return ctypes.CDLL(out)
 
 
-def check_order(lib, heads, group, batch, ragged=2, chunks=1, live=1 << 20, slots=512, proj=0,
-                qtiles=3):
+def check_order(lib, heads, group, batch, ragged=2, chunks=1, live=1 << 20, slots=512, windowed=0,
+                proj=0, qtiles=3):
     form = (ctypes.c_int * 4)()
     rc = lib.check(heads, group, batch, ragged, chunks, ctypes.c_long(live),
-                   ctypes.c_long(slots), proj, qtiles, form)
-    assert rc == 0, (heads, group, batch, ragged, chunks, live, proj, qtiles)
+                   ctypes.c_long(slots), windowed, proj, qtiles, form)
+    assert rc == 0, (heads, group, batch, ragged, chunks, live, windowed, proj, qtiles)
     return dict(zip(("lanes", "pair_heads", "xcds", "turn"), form))
 
 
@@ -69,8 +69,8 @@ def test_every_place_once(lib):
         group = rng.choice([1, 1, 2, 3, 4, 4, 5, 6, 7, 8, 12, 16, 20, 32])
         heads = group * rng.choice([1, 1, 2, 2, 3, 4, 5, 8, 16])
         f = check_order(lib, heads, group, rng.randint(1, 40), rng.randint(0, 2),
-                        rng.choice([1, 1, 1, 2, 5]), rng.choice([0, 511, 512, 5000]), 512,
-                        rng.randint(0, 1), rng.randint(1, 9))
+                        rng.choice([1, 1, 1, 2, 5]), rng.choice([0, 300, 511, 512, 5000]), 512,
+                        rng.randint(0, 1), rng.randint(0, 1), rng.randint(1, 9))
         forms.add((f["lanes"], f["pair_heads"] > 0, f["xcds"], f["turn"]))
     # linear, turned, pairs, spread over 8 / 4 / 2 / 1 XCDs
     assert forms == {(0, False, 0, 0), (0, False, 0, 1), (3, True, 0, 0), (3, False, 8, 1),
@@ -94,6 +94,13 @@ def test_every_place_once(lib):
     (8, 4, 16, dict(live=440, slots=256, proj=1, ragged=1), dict(lanes=3, pair_heads=2)),
     (8, 4, 64, dict(live=600, qtiles=1), dict(lanes=3, pair_heads=2)),
     (24, 6, 64, dict(live=5000), dict(lanes=3, pair_heads=4)),
+    (8, 4, 9, dict(live=224, windowed=1), dict(lanes=3, xcds=4, turn=1)),
+    (6, 3, 9, dict(live=224, windowed=1), dict(lanes=3, xcds=4, turn=1)),
+    (8, 2, 9, dict(live=5000, windowed=1), dict(lanes=0, turn=0)),
+    (8, 4, 9, dict(live=223, windowed=1), dict(lanes=0, turn=0)),
+    (8, 4, 9, dict(live=300, windowed=1, slots=256, proj=1), dict(lanes=0, turn=0)),
+    (8, 1, 6, dict(live=0, ragged=1), dict(lanes=0, turn=1)),   # eight kv heads of one head
+    (4, 1, 6, dict(live=511), dict(lanes=3, pair_heads=4)),
     (16, 4, 10, dict(live=319, slots=256, proj=1), dict(lanes=3, pair_heads=4)),
     (4, 4, 12, dict(live=600), dict(lanes=3, xcds=8, turn=1)),
     (4, 4, 7, dict(live=600), dict(lanes=0, turn=0)),          # fewer sequences than XCDs
