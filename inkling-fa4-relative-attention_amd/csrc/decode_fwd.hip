@@ -778,8 +778,17 @@ decode_stream_kernel(DecodeParams p) {
     mx = max_xor16(mx);
     mx = max_xor32(mx);
 
-    const float m_cand = fmaxf(m_run, mx);
-    const bool grow = m_cand > m_run + kRescaleThreshold;
+    // The base of the exponents.  The stream pass keeps it until the maximum has grown
+    // by the threshold.  The one-launch form takes each step's own maximum (unless that
+    // is as far below the base), whose weight is then exact in the 16 bits of P: its
+    // waves hold two to four steps where the stream's held one or two, and with one base
+    // for all of them the error of a windowed call grew by 3% (2.22e-3 -> 2.29e-3 in
+    // bf16).  The base falls by up to the threshold a step, in a wave's first four steps
+    // only (all it has, unless max_seqlen_k was too small): sums stay far inside fp32.
+    const float m_cand = kNw > 0 ? mx : fmaxf(m_run, mx);
+    const bool grow = kNw == 0 ? m_cand > m_run + kRescaleThreshold
+                               : m_cand > m_run || (cu.step < 4 * kNw && m_cand < m_run &&
+                                                    m_cand > m_run - kRescaleThreshold);
     const bool any_grow = wave_any(grow);
     float alpha = 1.f;
     if (any_grow) {

@@ -108,6 +108,38 @@ def test_short_rows_without_exactly_one_query(cuda):
     assert torch.equal(out[2], ref[0][2]) and torch.equal(lse[:, 2], ref[1][:, 2])
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_short_windows_keep_the_rounding_of_one_step(cuda, dtype):
+    # The error against fp64 is that of rounding each 32-key step's weights, relative to the
+    # step's largest, and the output to 16 bits: emulated here on the same numbers, so the two
+    # differ by fp32 rounding only (1%: with one base for a wave's steps it was 3% above).
+    lens = [520 + 83 * i for i in range(24)]
+    case = testing.make_case("short_round", [1] * 24, lens, 8, 2, 128, dtype, seed=11,
+                             window_left=511, rel_table=False, rel_extent=512, rel_dtype=dtype,
+                             scale=1 / 128)
+    print(f"rounding of windowed short decode, {dtype}", flush=True)
+    c = case.to(cuda)
+    out = inkling_fa4_rel_attention_decode(*c.args(), causal=True, window_size=(511, 0),
+                                           softmax_scale=c.scale, bottom_right=True).cpu().double()
+    want, rounded, ks = torch.zeros_like(out), torch.zeros_like(out), 0
+    for b, n in enumerate(lens):
+        lo = n - 512
+        k, v = (x[ks + lo:ks + n].double() for x in (case.k, case.v))
+        ks += n
+        for h in range(8):
+            x = k[:, h // 4] @ case.q[b, h].double() / 128 + case.rel[b, h].double().flip(0)
+            p = torch.exp(x - x.max())
+            want[b, h] = p @ v[:, h // 4] / p.sum()
+            step = torch.arange(lo, n) // 32 - lo // 32  # steps start at multiples of 32 keys
+            top = torch.full((int(step[-1]) + 1,), -torch.inf, dtype=torch.float64)
+            top = top.scatter_reduce(0, step, p, "amax")[step]
+            p16 = (p / top).to(dtype).double() * top
+            rounded[b, h] = (p16 @ v[:, h // 4] / p.sum()).to(dtype).double()
+    err, bound = (float((y - want).norm() / want.norm()) for y in (out, rounded))
+    assert err < 1.01 * bound, (err, bound)
+
+
 # (waves per workgroup, keys per wave) that the tile query reports: the one-launch form on
 # both sides of its rule, and the persistent waves
 @pytest.mark.parametrize("batch,keys,hq,hkv,window,waves,chunk", [
