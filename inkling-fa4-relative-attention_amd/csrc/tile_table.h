@@ -125,12 +125,11 @@ inline bool decode_pairs(bool fp8, int64_t head_dim, int64_t kv_heads, int64_t g
 // steps a wave (a window of 512 keys is 17 steps), and up to four where the
 // segments alone fill the chip.  Two passes -> one launch (one box, us, Hq 8 /
 // Hkv 2, d 128; sequences x keys):
-//   bf16 1 x 512 14.1 -> 10.8, 64 x 512 18.2 -> 12.3, 128 x 256 20.0 -> 11.0, 128 x
-//   512 26.5 -> 15.3, 64 x 1024 24.7 -> 18.9, 128 x 1024 39.6 -> 25.4, but 16 x 1024
-//   14.1 -> 16.2, 16 x 2048 16.2 -> 27.0;
-//   paged 64 x 512 19.0 -> 13.5, paged fp8 64 x 512 18.2 -> 14.1, window 511 over
-//   200..6000 paged keys 24 sequences 15.9 -> 14.0, 64 20.8 -> 15.0; window 1023
-//   (33 steps) 16.9 -> 21.1.
+//   bf16 1 x 300..600 14.2 -> 9.0, 64 x 300..600 18.3 -> 12.6, 128 x 100..200 16.5 -> 8.8,
+//   128 x 512 26.5 -> 15.3, 64 x 500..1000 22.3 -> 18.8, 128 x 1024 39.6 -> 25.4, but 16 x
+//   1024 14.1 -> 16.2, 16 x 2048 16.2 -> 27.0;
+//   paged 64 x 250..500 18.1 -> 13.4, fp8 18.0 -> 13.9, window 511 over 200..6000 paged
+//   keys 24 sequences 15.8 -> 14.2, 64 20.8 -> 15.2; window 1023 (33 steps) 16.9 -> 21.1.
 // With 4 waves a segment everything but 64 x 256 is slower (64 x 512 13.4, windows 18.5).
 // Groups above 8 take half the waves: their Q rows and tiles fill the LDS.
 constexpr int64_t decode_whole_waves(int64_t group) { return group > 8 ? 4 : 8; }
@@ -364,7 +363,7 @@ constexpr int64_t kWindowMinChunk = 4;
 // every query (the causal mask takes max_q keys at most).  With a window the
 // ranges are short wherever the queries sit: counting them so (instead of the
 // whole cache, us on one box): 3 x 300..500 queries, window 511, over 100..4000
-// keys 38.3 -> 26.3, 1 x 1000 32.9 -> 24.7, 6 x 20..40 22.5 -> 15.3.
+// keys 37.7 -> 27.3, 1 x 1000 32.9 -> 23.1, 6 x 20..40 21.9 -> 15.3.
 // no_prune: masked tiles are visited too (debug).  forced_chunk > 0: split every query
 // tile into chunks of that many tiles.  table: the bias is a shared table.
 inline PrefillSplit prefill_split_for(int64_t batch, int64_t n_heads, int64_t max_q,
